@@ -396,21 +396,37 @@ __global__ __launch_bounds__(kLgThreads, 2) void gemm1_large_kernel(Problem pb, 
   }
 }
 
-// ------------------------------------------------------------------------------ GEMM1, 128-row m-blocks
-// For the 128-row blocks over an expert's class 0 and 1 rows.  A workgroup of 8 wavefronts (one
-// per CU, two per SIMD, 148 KB of LDS) owns one unit = (m-block, 128 C columns = 256 weight rows,
-// 128 up and 128 gate) and stages BOTH operands of each K-block through a 3-stage LDS ring by
-// DMA: the weight rows are read once per unit and shared by the block's 128 rows (the
-// per-wavefront weight streams above re-read them per 64 rows through the vector-memory path).
-// Wavefront w = (wm, wn) = (w % 2, w / 2) computes rows 64 wm .. 64 wm + 63 x its 64 weight rows
-// (C columns 32 wn .. 32 wn + 31, up and gate): 4 x 4 MFMA 16x16x128 tiles per K-block, 64
-// accumulator registers, so that the two wavefronts of a SIMD hide each other's MFMA and LDS
-// latencies.
+// ------------------------------------------------------------------------------ GEMM1, LDS-staged m-blocks
+// For the blocks of up to 160 rows over an expert's class 0 and 1 rows.  A workgroup of 8 wavefronts
+// (one per CU, two per SIMD, 158 KB of LDS) owns one unit = (m-block, 128 C columns = 256 weight
+// rows, 128 up and 128 gate) and stages BOTH operands of each K-block through a 3-stage LDS ring by
+// DMA.  Wavefront w = (wm, wn) = (w / 4, w % 4) computes the tokens of half wm of the block's m-tiles x
+// its 64 weight rows (C columns 32 wn .. 32 wn + 31, up and gate).  The two wavefronts of a SIMD are the
+// two halves of the same columns, so an odd m-tile count loads no SIMD more than another.
+//
+// The weights are the MFMA's first operand: a lane's four results are four weight rows of one token, so
+// the block scale is one factor per m-tile and weight half instead of four, a token's row scale is one
+// 4-byte LDS read instead of a 16-byte one, and with the weight rows ordered for it (bg_wrow) a lane ends
+// with 8 consecutive C columns of its token: one 16-byte store per f16 term instead of eight 2-byte ones.
+//
+// K loop.  An MFMA's products are scaled and accumulated one phase (the four MFMAs of an m-tile) later,
+// so no FMA waits for the MFMA before it; fresh fp8 MFMAs with four such FMAs each issue at 95% of the
+// MFMAs alone, one or two wavefronts per SIMD, where FMAs that follow their own MFMA reach half of it
+// with one and 85% with two (measured).  Operands are read one phase ahead: the next m-tile's rows, and
+// in the last phase of a K-block the next K-block's weights and first m-tile, which is why the barrier
+// that publishes stage j + 1 (and frees stage j) stands before the last phase of K-block j.  The DMAs of
+// stage j + 3 are spread evenly over the phases that follow it: each takes the address unit ~16 cycles,
+// and the 56-64 of a stage issued together held every wavefront for ~890 cycles of a 2432-cycle K-block.
+// With the balanced blocks (row_blocks) GEMM1 went 425 -> 369 us at T = 8192, 572 -> 494 at 14107 and
+// 256 -> 229 at 5000 (even, even and zipf routing); a K-block of a 160-row block takes ~2140 cycles at the
+// ~1.95 GHz that the card keeps under this load, of which its MFMAs need 1300.  Without the DMAs it is ~1830,
+// with W13 served from L2 15% less: what is left is the barrier of every K-block and the operand reads
+// behind it, the DMAs' latency and the clock.
 //
 // The DMAs and their wait are inline asm and the LDS operand reads ordinary loads: the compiler
-// schedules the reads with exact lgkmcnt waits and never drains the DMAs before them.
+// waits for the reads with exact lgkmcnt counts and never drains the DMAs before them.
 //
-// LDS stage: A [128 rows][128 B], B [256 rows][128 B], 128 row scales.  A row's 16-byte chunk c
+// LDS stage: A [160 rows][128 B], B [256 rows][128 B], 160 row scales.  A row's 16-byte chunk c
 // sits in slot c ^ slot_key8(row): a DMA instruction writes 8
 // rows x 8 slots in lane order (each lane fetching the chunk that belongs in its slot, 8 lanes
 // per 128-byte row segment), and an MFMA operand read (16 rows, two chunks per lane) puts any 16
@@ -418,21 +434,18 @@ __global__ __launch_bounds__(kLgThreads, 2) void gemm1_large_kernel(Problem pb, 
 // ones of a 128-byte row).
 constexpr int kBgWaves = 8;
 constexpr int kBgThreads = 64 * kBgWaves;
-constexpr int kBgRows = 128;
 constexpr int kBgWRows = 256;
 constexpr int kBgStages = 3;
-constexpr int kBgA = kBgRows * 128;
+constexpr int kBgA = kBigRows * 128;
 constexpr int kBgB = kBgWRows * 128;
-constexpr int kBgStage = kBgA + kBgB + kBgRows * 4;
-constexpr int kBgOps = 2 + 4 + 1;            // per wavefront and K-block: A, B and row-scale DMAs
+constexpr int kBgStage = kBgA + kBgB + kBigRows * 4;
 
-// LDS row R of a 128-row unit -> row of the permuted pairs.  Regular blocks: R < rows.  A mixed
+// LDS row R of a unit -> row of the permuted pairs.  Regular blocks: R < rows.  A mixed
 // block (an expert's last regular block with its <= 32 exact-product rows folded in) puts its
 // regular rows at LDS rows [0, cap) and its exact rows at [cap, 128), cap = 128 - 16 ceil(x / 16);
-// the exact rows follow the regular ones in the permuted order.  Rows from xfrom on (0 for an
-// exact-product block, cap for a mixed one, 128 otherwise) get exact products and an f16 lo term.
+// the exact rows follow the regular ones in the permuted order.
 struct RowMap {
-  int row0, rows, cap, xrows, xfrom;
+  int row0, rows, cap, xrows;
   __device__ __forceinline__ int src(int R) const {
     return R < cap ? row0 + min(R, rows - 1) : row0 + rows + min(R - cap, xrows - 1);
   }
@@ -440,359 +453,350 @@ struct RowMap {
 };
 __device__ __forceinline__ RowMap row_map(int row0, int rows, int flags) {
   if (flags & kFlagMixed) {
-    const int x = flags >> kMixedShift, cap = kBgRows - 16 * ((x + 15) / 16);
-    return RowMap{row0, rows, cap, x, cap};
+    const int x = flags >> kMixedShift, cap = kMixedRows - 16 * ((x + 15) / 16);
+    return RowMap{row0, rows, cap, x};
   }
-  return RowMap{row0, rows, kBgRows, 0, (flags & kFlagExactProducts) ? 0 : kBgRows};
+  return RowMap{row0, rows, kBigRows, 0};
 }
 
-// A mixed block's m-tiles for wavefront half wm: nf regular tiles from tf0 and nx exact tiles from
-// tx0.  An exact tile costs about three regular ones, so with two exact tiles each half takes one
-// of them and half of the regular tiles, and with one the other half takes more regular tiles.
+// The m-tiles of wavefront half wm: nf tiles on the e4m3 MFMA from tf0 and nx (0 or 1) exact tiles from
+// tx0.  A mixed block's exact tile costs about three regular ones, so with two exact tiles each half takes
+// one of them and half of the regular tiles, and with one the other half takes more regular tiles.
 struct TileSplit {
   int nf, nx, tf0, tx0;
 };
-__device__ __forceinline__ TileSplit mixed_split(const RowMap& rm, int wm) {
+__device__ __forceinline__ TileSplit tile_split(const RowMap& rm, int flags, int wm) {
   const int nr = (rm.rows + 15) / 16;
-  if (rm.cap == kBgRows - 32) {
-    const int a = (nr + 1) / 2;
-    return wm == 0 ? TileSplit{a, 1, 0, 6} : TileSplit{nr - a, 1, a, 7};
+  if (flags & kFlagMixed) {
+    if (rm.cap == kMixedRows - 32) {
+      const int a = (nr + 1) / 2;
+      return wm == 0 ? TileSplit{a, 1, 0, 6} : TileSplit{nr - a, 1, a, 7};
+    }
+    const int a = min(min(nr, 4), (nr + 4) / 2);
+    return wm == 0 ? TileSplit{a, 0, 0, 0} : TileSplit{nr - a, 1, a, 7};
   }
-  const int a = min(min(nr, 4), (nr + 4) / 2);
-  return wm == 0 ? TileSplit{a, 0, 0, 0} : TileSplit{nr - a, 1, a, 7};
+  if (flags & kFlagExactProducts) return TileSplit{0, wm < nr ? 1 : 0, 0, wm};
+  const int a = (nr + 1) / 2;
+  return wm == 0 ? TileSplit{a, 0, 0, 0} : TileSplit{nr - a, 0, a, 0};
 }
 
-// One unit.  Wavefront (wm, wn) computes m-tiles NT wm .. NT wm + NT - 1: NT = 4 for blocks of more
-// than 64 rows, 2 for 33..64 rows and 1 for at most 32 (the short last blocks of an expert's
-// classes cost a quarter of the MFMA and VALU work of a full one).  kExact (blocks of at most 32
-// exact-product rows, NT = 1): the f16 MFMA on operands widened exactly, and C's lo term in f16.
-// kOnce: the block is its expert's only one, so each weight line is read once per call, by one
-// DMA instruction (8 lanes x 16 B), and its DMAs carry the non-temporal hint: 5% less GEMM1
-// time at 1024 tokens (about one block per expert), measured.  Experts with several blocks keep
-// ordinary DMAs, which let the blocks share the weights through L2 (the hint on every block cost
-// 20% at 8192 tokens, measured).  A template parameter, not a branch: the branch in the K loop
-// cost up to 4% on the other blocks, measured.
-template <int NT, bool kExact, bool kOnce>
+// Weight row of LDS row R (0..255) of a unit, relative to the unit's first up row: group R / 64 of 32 C
+// columns, n-tile (R / 16) % 4 (0, 1 up, 2, 3 gate), MFMA row m = R % 16, which is C column
+// 8 (m / 4) + 4 (n % 2) + m % 4 of the group, so that a lane (MFMA rows 4 kg .. 4 kg + 3 of both n-tiles)
+// holds columns 8 kg .. 8 kg + 7.
+__device__ __forceinline__ int bg_wrow(int R, int I) {
+  const int n = (R >> 4) & 3, m = R & 15;
+  return (n < 2 ? 0 : I) + 32 * (R >> 6) + 8 * (m >> 2) + 4 * (n & 1) + (m & 3);
+}
+
+// One DMA of K-block stage j, if j < end: to LDS address lds + at, from the wave-uniform base plus the lane's
+// byte offset.  The branch is inside the asm: the K loop around it stays straight-line code, so the
+// compiler's schedule and its MFMA wait states do not see it.
+#define MOEFP8_DMA_IF(PRE, OP, SUFFIX, POST, ...)                                                               \
+  asm volatile("s_cmp_lt_i32 %4, %5\n\ts_cbranch_scc0 .Ldma_skip%=\n\t" PRE "s_add_u32 m0, %2, %3\n\ts_nop 0\n\t" OP \
+               " %0, %1" SUFFIX POST "\n.Ldma_skip%=:"                                                          \
+               : : "v"(voff), "s"(sbase), "s"(lds), "s"(at), "s"(j), "s"(end), ##__VA_ARGS__ : "memory", "m0", "scc")
+__device__ __forceinline__ void dma_lds16_if(uint32_t voff, const void* sbase, uint32_t lds, uint32_t at, int j, int end) {
+  MOEFP8_DMA_IF("", "global_load_lds_dwordx4", "", "");
+}
+__device__ __forceinline__ void dma_lds16_if_nt(uint32_t voff, const void* sbase, uint32_t lds, uint32_t at, int j, int end) {
+  MOEFP8_DMA_IF("", "global_load_lds_dwordx4", " nt", "");
+}
+// The same with execution mask {lo, hi} (all lanes, some, or none: with none the instruction counts and
+// completes without reading or writing anything, so that every wavefront has the same number of operations
+// in flight, whichever rows it carries).  All lanes are active before and after.
+#define MOEFP8_EXEC_SET "s_mov_b32 exec_lo, %6\n\ts_mov_b32 exec_hi, %7\n\t"
+#define MOEFP8_EXEC_ALL "\n\ts_mov_b64 exec, -1"
+__device__ __forceinline__ void dma_lds16_if_m(uint32_t voff, const void* sbase, uint32_t lds, uint32_t at, int j, int end,
+                                               int lo, int hi) {
+  MOEFP8_DMA_IF(MOEFP8_EXEC_SET, "global_load_lds_dwordx4", "", MOEFP8_EXEC_ALL, "s"(lo), "s"(hi));
+}
+__device__ __forceinline__ void dma_lds4_if_m(uint32_t voff, const void* sbase, uint32_t lds, uint32_t at, int j, int end,
+                                              int lo, int hi) {
+  MOEFP8_DMA_IF(MOEFP8_EXEC_SET, "global_load_lds_dword", "", MOEFP8_EXEC_ALL, "s"(lo), "s"(hi));
+}
+// This wavefront's LDS reads are complete and at most N of its DMAs in flight (none from K-block `last` on, where
+// no further stage has been started), then the workgroup barrier.
+template <int N>
+__device__ __forceinline__ void publish_stage(int j = 0, int last = 1) {
+  asm volatile("s_cmp_lt_i32 %1, %2\n\ts_cbranch_scc1 .Lmore%=\n\ts_waitcnt vmcnt(0)\n.Lmore%=:\n\t"
+               "s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N), "s"(j), "s"(last) : "memory", "scc");
+}
+// All ones where x < y, else 0 (x, y wave-uniform, |x - y| < 2^31).  In asm: the compiler would turn it into a
+// vector select, whose result no scalar operand takes.
+__device__ __forceinline__ int mask_less(int x, int y) {
+  int m;
+  asm("s_sub_i32 %0, %1, %2\n\ts_ashr_i32 %0, %0, 31" : "=s"(m) : "s"(x), "s"(y) : "scc");
+  return m;
+}
+
+// One unit: this wavefront's NF m-tiles from tf0 on the e4m3 MFMA and NX (0 or 1) m-tile at tx0 with exact
+// products (the f16 MFMA on operands widened exactly).  KA: activation DMAs per wavefront and stage (8
+// rows each, 64 rows per step of KA over the 8 wavefronts).  kOnce: the block is its expert's only one, so
+// each weight line is read once per call, by one DMA instruction (8 lanes x 16 B), and its DMAs carry
+// the non-temporal hint: 5% less GEMM1 time at 1024 tokens (about one block per expert), measured.
+// Experts with several blocks keep ordinary DMAs, which let the blocks share the weights through L2
+// (the hint on every block cost 20% at 8192 tokens, measured).
+template <int NF, int NX, int KA, bool kOnce>
 __device__ __forceinline__ void gemm1_big_unit(const Problem& pb, const Plan& pl, const CHalf8& ch, uint8_t* ring,
-                                               uint32_t ring_lds, uint32_t sink_lds, const float2* sw_s,
-                                               float (*amax_s)[kBgRows],
-                                               int e, int row0, int rows, int cb, int* next_s, int n_units) {
-  static_assert(NT == 1 || NT == 2 || NT == 4, "m-tiles per wavefront");
-  static_assert(!kExact || NT == 1, "exact-product blocks hold at most 32 rows");
-  const int H = pb.H, I = pb.I, T = pb.T, KB = H / kBlock, NCB = I / kBlock;
-  const int wave = wave_index(), lane = lane_id(), lr = lane & 15, kg = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
-  // DMA lane roles: row (lane / 8) of an 8-row group, slot lane % 8
-  const int drow = lane >> 3, dslot = lane & 7;
-  // operand read offsets inside a 16-row tile (swizzled chunks 2kg and 2kg + 1 of row lr)
-  const int rd0 = lr * 128 + (((2 * kg) ^ slot_key8(lr)) * 16);
-  const int rd1 = lr * 128 + (((2 * kg + 1) ^ slot_key8(lr)) * 16);
-  // DMA sources as per-lane byte offsets from wave-uniform bases: A rows 16w + 8q + drow (the
-  // tokens' hidden rows, clamped to the block), B LDS rows 32w + 8q + drow (LDS row R holds n-tile
-  // (R % 64) / 16 of weight-row group R / 64: 0, 1 up, 2, 3 gate), row scales of rows 64 (w % 2) + lane
-  uint32_t aoff[2], boff[4];
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int r = 16 * wave + 8 * q + drow;
-    const int tok = clamp_index(pl.perm_token[row0 + min(r, rows - 1)], T);
-    aoff[q] = (uint32_t)tok * (uint32_t)H + (uint32_t)((dslot ^ slot_key8(r)) * 16);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int R = 32 * wave + 8 * q + drow;
-    const int g = R >> 6, n = (R >> 4) & 3, rr = R & 15;
-    const int wrow = (n < 2 ? 0 : I) + cb * kBlock + 32 * g + 16 * (n & 1) + rr;
-    boff[q] = (uint32_t)wrow * (uint32_t)H + (uint32_t)((dslot ^ slot_key8(R)) * 16);
-  }
-  const uint32_t soff =
-      wave < 2 ? 4u * (uint32_t)clamp_index(pl.perm_token[row0 + min(64 * (wave & 1) + lane, rows - 1)], T) : 0u;
-  const uint8_t* wbase = pb.w13 + (size_t)e * 2 * I * H;
-  auto issue = [&](int j) {
-    const int k = min(j, KB - 1);
-    const uint32_t st = ring_lds + (uint32_t)((j % kBgStages) * kBgStage);
-    const uint8_t* abase = pb.hidden + (size_t)k * kBlock;
-    const uint8_t* bbase = wbase + (size_t)k * kBlock;
-    const float* sbase = pb.hscale + (size_t)k * T;
-#pragma unroll
-    for (int q = 0; q < 2; q++) dma_lds16_s(aoff[q], abase, st + (16 * wave + 8 * q) * 128);
-    if (kOnce) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) dma_lds16_s_nt(boff[q], bbase, st + kBgA + (32 * wave + 8 * q) * 128);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; q++) dma_lds16_s(boff[q], bbase, st + kBgA + (32 * wave + 8 * q) * 128);
-    }
-    // every wavefront issues the same operations: wavefronts 0 and 1 DMA the row scales of rows
-    // 64 w + lane, 2..7 one 4-byte word (one line, all lanes) into a sink: GEMM1 -3 / -4 to -8 µs
-    // at T = 1024 / 8192 against all eight DMAing the 64 scattered scales of 0 and 1 (measured)
-    dma_lds4_s(soff, sbase, wave < 2 ? st + kBgA + kBgB + (wave & 1) * 256 : sink_lds);
-  };
-
-  // the table and scale loads of the unit are complete: only DMAs count from here
-  MOEFP8_WAIT_VMCNT(0);
-  for (int d = 0; d < kBgStages - 1; d++) issue(d);
-  v4f acc[NT][4];
-#pragma unroll
-  for (int i = 0; i < NT; i++)
-#pragma unroll
-    for (int n = 0; n < 4; n++) acc[i][n] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  for (int j = 0; j < KB; j++) {
-    // stage j's DMAs are done once only the following stage's (7 per wavefront) may be in flight
-    static_assert((kBgStages - 2) * kBgOps == 7, "wait count");
-    MOEFP8_WAIT_VMCNT(7);
-    barrier_lds();
-    const uint8_t* st = ring + (j % kBgStages) * kBgStage;
-    v8i B[4];
-#pragma unroll
-    for (int n = 0; n < 4; n++) {
-      const uint8_t* bt = st + kBgA + (64 * wn + 16 * n) * 128;
-      B[n] = cat(*reinterpret_cast<const v4i*>(bt + rd0), *reinterpret_cast<const v4i*>(bt + rd1));
-    }
-    const float2 sw = sw_s[j];
-#pragma unroll
-    for (int i = 0; i < NT; i++) {
-      const int t = NT * wm + i;
-      const uint8_t* at = st + t * 16 * 128;
-      const v8i a = cat(*reinterpret_cast<const v4i*>(at + rd0), *reinterpret_cast<const v4i*>(at + rd1));
-      const float4 sa = *reinterpret_cast<const float4*>(st + kBgA + kBgB + (16 * t + 4 * kg) * 4);
-      const float4 su = {sa.x * sw.x, sa.y * sw.x, sa.z * sw.x, sa.w * sw.x};
-      const float4 sg = {sa.x * sw.y, sa.y * sw.y, sa.z * sw.y, sa.w * sw.y};
-      v8h a16[4];
-      if constexpr (kExact) widen_fp8_operand(a, a16);
-#pragma unroll
-      for (int n = 0; n < 4; n++) {
-        const float4 sc = n < 2 ? su : sg;
-        v4f p;
-        if constexpr (kExact) {
-          v8h b16[4];
-          widen_fp8_operand(B[n], b16);
-          p = mfma_f16_block(a16, b16, v4f{0.f, 0.f, 0.f, 0.f});
-        } else {
-          p = mfma16x16x128(a, B[n], v4f{0.f, 0.f, 0.f, 0.f});
-        }
-        acc[i][n][0] += p[0] * sc.x;
-        acc[i][n][1] += p[1] * sc.y;
-        acc[i][n][2] += p[2] * sc.z;
-        acc[i][n][3] += p[3] * sc.w;
-      }
-    }
-    // stage (j + 2) % 3 was last read at step j - 1, before this step's barrier
-    issue(j + kBgStages - 1);
-  }
-  MOEFP8_WAIT_VMCNT(0);
-  // the workgroup's next unit, claimed now so that the atomic overlaps the epilogue
-  if (threadIdx.x == 0) *next_s = grab_unit(pl.queues, n_units);
-
-  // epilogue: C = silu(gate) * up, per-row max over the unit's 128 columns, hi/lo split
-  const int col0 = cb * kBlock + 32 * wn;
-  float c[NT][2][4];
-#pragma unroll
-  for (int i = 0; i < NT; i++)
-#pragma unroll
-    for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) c[i][jn][r] = silu_f32(acc[i][jn + 2][r]) * acc[i][jn][r];
-#pragma unroll
-  for (int i = 0; i < NT; i++) {
-    const int t = NT * wm + i;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float m = fmaxf(fabsf(c[i][0][r]), fabsf(c[i][1][r]));
-      m = fmaxf(m, dpp_f32<kDppXor1>(m));
-      m = fmaxf(m, dpp_f32<kDppXor2>(m));
-      m = fmaxf(m, dpp_f32<kDppHalfMirror>(m));
-      m = fmaxf(m, dpp_f32<kDppRowMirror>(m));
-      if (lr == 0) amax_s[wn][16 * t + 4 * kg + r] = m;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NT; i++) {
-    const int t = NT * wm + i;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = 16 * t + 4 * kg + r;
-      if (row >= rows) continue;
-      const float amax = fmaxf(fmaxf(amax_s[0][row], amax_s[1][row]), fmaxf(amax_s[2][row], amax_s[3][row]));
-      float inv, scale;
-      split_scale(amax, inv, scale);
-      const size_t p = (size_t)(row0 + row);
-#pragma unroll
-      for (int jn = 0; jn < 2; jn++) store_c(ch, p, I, col0 + 16 * jn + lr, c[i][jn][r], inv);
-      if (wn == 0 && lr == 0) ch.scale[p * NCB + cb] = scale;
-    }
-  }
-}
-
-// One unit of a mixed block.  This wavefront computes NF m-tiles tf0 .. tf0 + NF - 1 on the e4m3
-// MFMA and NX m-tiles tx0 .. tx0 + NX - 1 with exact products (the f16 MFMA on operands widened
-// exactly), its half of the block's tiles (mixed_split); every wavefront issues the same DMAs and
-// barriers.  (Kept apart from gemm1_big_unit: the compiler schedules the regular blocks' K loop
-// worse in this general form, LDS reads no longer hoisted ahead of the MFMAs, ~10% slower.)
-template <int NF, int NX>
-__device__ __forceinline__ void gemm1_big_mixed_unit(const Problem& pb, const Plan& pl, const CHalf8& ch, uint8_t* ring,
-                                               uint32_t ring_lds, uint32_t sink_lds, const float2* sw_s,
-                                               float (*amax_s)[kBgRows],
-                                               int e, const RowMap& rm, int cb, int tf0, int tx0, int* next_s,
-                                               int n_units) {
+                                               uint32_t ring_lds, int e, const RowMap& rm, int cb, int tf0, int tx0,
+                                               int* next_s, int n_units) {
   constexpr int NT = NF + NX;
-  static_assert(NT >= 1 && NT <= 4, "m-tiles per wavefront");
+  constexpr int kOps = KA + 4 + 1;   // DMAs per wavefront and stage: A, B, row scales
+  static_assert(NT <= 5 && NX <= 1 && KA >= 1 && KA <= 3, "m-tiles per wavefront");
   const int H = pb.H, I = pb.I, T = pb.T, KB = H / kBlock, NCB = I / kBlock;
-  const int wave = wave_index(), lane = lane_id(), lr = lane & 15, kg = lane >> 4;
-  const int wn = wave >> 1;
+  int lane = lane_id();
+  asm volatile("" : "+v"(lane));   // (addresses formed per unit, not kept across units)
+  const int wave = wave_index(), lr = lane & 15, kg = lane >> 4;
+  const int wn = wave & 3;
   auto tile = [&](int i) { return i < NF ? tf0 + i : tx0 + (i - NF); };
   // DMA lane roles: row (lane / 8) of an 8-row group, slot lane % 8
   const int drow = lane >> 3, dslot = lane & 7;
-  // operand read offsets inside a 16-row tile (swizzled chunks 2kg and 2kg + 1 of row lr)
-  const int rd0 = lr * 128 + (((2 * kg) ^ slot_key8(lr)) * 16);
-  const int rd1 = lr * 128 + (((2 * kg + 1) ^ slot_key8(lr)) * 16);
-  // DMA sources as per-lane byte offsets from wave-uniform bases: A rows 16w + 8q + drow (the
-  // tokens' hidden rows), B LDS rows 32w + 8q + drow (LDS row R holds n-tile (R % 64) / 16 of
-  // weight-row group R / 64: 0, 1 up, 2, 3 gate), row scales of rows 64 (w % 2) + lane
-  uint32_t aoff[2], boff[4];
+  // DMA sources as per-lane byte offsets from wave-uniform bases: A rows 8 (w + 8q) + drow (the
+  // tokens' hidden rows), B LDS rows 32w + 8q + drow, row scales of rows 64 (7 - w) + lane
+  uint32_t aoff[KA], boff[4];
+  int am[KA];
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int r = 16 * wave + 8 * q + drow;
+  for (int q = 0; q < KA; q++) {
+    const int r0 = 8 * (wave + 8 * q), r = r0 + drow;
     const int tok = clamp_index(pl.perm_token[rm.src(r)], T);
     aoff[q] = (uint32_t)tok * (uint32_t)H + (uint32_t)((dslot ^ slot_key8(r)) * 16);
+    // (groups without a row of the block are not fetched: what the LDS holds there reaches no stored row)
+    am[q] = mask_less(r0, rm.rows) | (mask_less(rm.cap - 1, r0) & mask_less(r0, rm.cap + rm.xrows));
   }
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     const int R = 32 * wave + 8 * q + drow;
-    const int g = R >> 6, n = (R >> 4) & 3, rr = R & 15;
-    const int wrow = (n < 2 ? 0 : I) + cb * kBlock + 32 * g + 16 * (n & 1) + rr;
-    boff[q] = (uint32_t)wrow * (uint32_t)H + (uint32_t)((dslot ^ slot_key8(R)) * 16);
+    boff[q] = (uint32_t)(cb * kBlock + bg_wrow(R, I)) * (uint32_t)H + (uint32_t)((dslot ^ slot_key8(R)) * 16);
   }
-  const uint32_t soff = wave < 2 ? 4u * (uint32_t)clamp_index(pl.perm_token[rm.src(64 * (wave & 1) + lane)], T) : 0u;
+  const int sgrp = kBgWaves - 1 - wave;
+  // (the stage holds kBigRows scales: the last group is cut to those)
+  // (the stage holds kBigRows scales: the last group is cut to those)
+  const int s_lo = mask_less(sgrp, KA) & mask_less(64 * sgrp, rm.xrows ? kMixedRows : rm.rows);
+  const int s_hi = s_lo & mask_less(64 * sgrp + 32, kBigRows);
+  static_assert(kBigRows % 32 == 0, "whole half-wavefronts of scales");
+  const int srow = min(64 * sgrp + lane, kBigRows - 1);
+  const uint32_t soff = 4u * (uint32_t)clamp_index(pl.perm_token[rm.src(srow)], T);
+  // the unit's weight scales of K-block l in lane l (up, gate; KB <= 64), read per K-block with readlane
+  const float* swp = pb.s13 + ((size_t)e * (2 * I / kBlock) + cb) * KB + min(lane, KB - 1);
+  float swu_v = swp[0], swg_v = swp[(size_t)NCB * KB];
   const uint8_t* wbase = pb.w13 + (size_t)e * 2 * I * H;
-  auto issue = [&](int j) {
-    const int k = min(j, KB - 1);
-    const uint32_t st = ring_lds + (uint32_t)((j % kBgStages) * kBgStage);
-    const uint8_t* abase = pb.hidden + (size_t)k * kBlock;
-    const uint8_t* bbase = wbase + (size_t)k * kBlock;
-    const float* sbase = pb.hscale + (size_t)k * T;
+
+  // op k of stage j's DMAs (k < 4: weight rows, then activation rows, then row scales) into the slot at
+  // LDS address st; past the last K-block nothing is fetched.  The bases move on with the stages.
+  const uint8_t *wb = wbase, *hb = pb.hidden;
+  const float* sb = pb.hscale;
+  auto issue_op = [&](int j, uint32_t st, int k) {
+    if (k < 4) {
+      const uint32_t at = kBgA + (32 * wave + 8 * k) * 128;
+      if (kOnce) dma_lds16_if_nt(boff[k], wb, st, at, j, KB);
+      else dma_lds16_if(boff[k], wb, st, at, j, KB);
+    } else if (k < 4 + KA) {
+      const uint32_t at = 8 * (wave + 8 * (k - 4)) * 128;
+      dma_lds16_if_m(aoff[k - 4], hb, st, at, j, KB, am[k - 4], am[k - 4]);
+    } else {
+      dma_lds4_if_m(soff, sb, st, kBgA + kBgB + sgrp * 256, j, KB, s_lo, s_hi);
+    }
+  };
+  auto next_stage = [&]() {
+    wb += kBlock;
+    hb += kBlock;
+    sb += T;
+  };
+  // the ops of a stage are spread over the 2 NT half phases from the last phase of K-block j - 3 on
+  constexpr int kParts = NT > 0 ? 2 * NT : 1;
+  auto issue_part = [&](int j, uint32_t slot, int part) {
 #pragma unroll
-    for (int q = 0; q < 2; q++) dma_lds16_s(aoff[q], abase, st + (16 * wave + 8 * q) * 128);
-#pragma unroll
-    for (int q = 0; q < 4; q++) dma_lds16_s(boff[q], bbase, st + kBgA + (32 * wave + 8 * q) * 128);
-    // every wavefront issues the same operations: wavefronts 0 and 1 DMA the row scales of rows
-    // 64 w + lane, 2..7 one 4-byte word (one line, all lanes) into a sink: GEMM1 -3 / -4 to -8 µs
-    // at T = 1024 / 8192 against all eight DMAing the 64 scattered scales of 0 and 1 (measured)
-    dma_lds4_s(soff, sbase, wave < 2 ? st + kBgA + kBgB + (wave & 1) * 256 : sink_lds);
+    for (int k = 0; k < kOps; k++)
+      if (k * kParts / kOps == part) issue_op(j, slot, k);
   };
 
-  // the table and scale loads of the unit are complete: only DMAs count from here
-  MOEFP8_WAIT_VMCNT(0);
-  for (int d = 0; d < kBgStages - 1; d++) issue(d);
-  v4f acc[NT][4];
-#pragma unroll
-  for (int i = 0; i < NT; i++)
-#pragma unroll
-    for (int n = 0; n < 4; n++) acc[i][n] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  for (int j = 0; j < KB; j++) {
-    // stage j's DMAs are done once only the following stage's (7 per wavefront) may be in flight
-    static_assert((kBgStages - 2) * kBgOps == 7, "wait count");
-    MOEFP8_WAIT_VMCNT(7);
-    barrier_lds();
-    const uint8_t* st = ring + (j % kBgStages) * kBgStage;
-    v8i B[4];
+  // operand read offsets inside a 16-row tile (swizzled chunks 2kg and 2kg + 1 of row lr)
+  const int rd0 = lr * 128 + (((2 * kg) ^ slot_key8(lr)) * 16);
+  const int rd1 = lr * 128 + (((2 * kg + 1) ^ slot_key8(lr)) * 16);
+  constexpr int NA = NT > 0 ? NT : 1;
+  v8i A[2], B[2][4];
+  float sa[2];
+  v4f acc[NA][4], p[2][4];
+  float su[2] = {0.f, 0.f}, sg[2] = {0.f, 0.f};
+  auto read_a = [&](const uint8_t* st, int i, int d) {
+    const uint8_t* at = st + tile(i) * 2048;
+    A[d] = cat(*reinterpret_cast<const v4i*>(at + rd0), *reinterpret_cast<const v4i*>(at + rd1));
+    sa[d] = *reinterpret_cast<const float*>(st + kBgA + kBgB + (16 * tile(i) + lr) * 4);
+  };
+  auto read_b = [&](const uint8_t* st, int d) {
 #pragma unroll
     for (int n = 0; n < 4; n++) {
       const uint8_t* bt = st + kBgA + (64 * wn + 16 * n) * 128;
-      B[n] = cat(*reinterpret_cast<const v4i*>(bt + rd0), *reinterpret_cast<const v4i*>(bt + rd1));
+      B[d][n] = cat(*reinterpret_cast<const v4i*>(bt + rd0), *reinterpret_cast<const v4i*>(bt + rd1));
     }
-    const float2 sw = sw_s[j];
+  };
+  auto retire = [&](int i, int d, int n) {   // scale and accumulate the products of m-tile i, n-tile n in p[d]
+    const float s = n < 2 ? su[d] : sg[d];
+#pragma unroll
+    for (int r = 0; r < 4; r++) acc[i][n][r] += p[d][n][r] * s;
+  };
+#pragma unroll
+  for (int i = 0; i < NA; i++)
+#pragma unroll
+    for (int n = 0; n < 4; n++) acc[i][n] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < 2; d++)
+#pragma unroll
+    for (int n = 0; n < 4; n++) p[d][n] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  // the table and scale loads of the unit are complete: only DMAs count from here
+  asm volatile("" : "+v"(swu_v), "+v"(swg_v));
+  MOEFP8_WAIT_VMCNT(0);
+#pragma unroll
+  for (int d = 0; d < 2; d++) {
+#pragma unroll
+    for (int k = 0; k < kOps; k++) issue_op(d, ring_lds + d * kBgStage, k);
+    next_stage();
+  }
+  constexpr int kFirst = NT > 0 ? (2 * kOps + kParts - 1) / kParts : kOps;   // ops of the first two parts
+  issue_part(2, ring_lds + 2 * kBgStage, 0);
+  if constexpr (NT > 0) issue_part(2, ring_lds + 2 * kBgStage, 1);
+  // stage 0 is there once only stage 1's and the started stage 2's DMAs may be in flight
+  publish_stage<kOps + kFirst>(1, KB - 1);
+  if constexpr (NT > 0) {
+    read_b(ring, 0);
+    read_a(ring, 0, 0);
+  }
+
+  uint32_t slot = 0;   // byte offset of K-block j's stage
+  auto kblock = [&](int j, auto parity) {
+    constexpr int q = decltype(parity)::value;
+    constexpr uint32_t kLast = (kBgStages - 1) * kBgStage;
+    const uint32_t slot1 = slot == kLast ? 0 : slot + kBgStage, slot2 = slot == 0 ? kLast : slot - kBgStage;
+    const uint8_t* st = ring + slot;
+    const uint8_t* st1 = ring + slot1;
+    const float swu = readlane_f32(swu_v, j), swg = readlane_f32(swg_v, j);
+    if constexpr (NT == 0) {
+      publish_stage<kOps>(j, KB - 2);
+      next_stage();
+      issue_part(j + 3, ring_lds + slot, 0);
+    }
 #pragma unroll
     for (int i = 0; i < NT; i++) {
-      const int t = tile(i);
-      const uint8_t* at = st + t * 16 * 128;
-      const v8i a = cat(*reinterpret_cast<const v4i*>(at + rd0), *reinterpret_cast<const v4i*>(at + rd1));
-      const float4 sa = *reinterpret_cast<const float4*>(st + kBgA + kBgB + (16 * t + 4 * kg) * 4);
-      const float4 su = {sa.x * sw.x, sa.y * sw.x, sa.z * sw.x, sa.w * sw.x};
-      const float4 sg = {sa.x * sw.y, sa.y * sw.y, sa.z * sw.y, sa.w * sw.y};
+      const int cur = (q * NT + i) & 1, nxt = cur ^ 1, prev = (i + NT - 1) % NT;
+      if (i == NT - 1) {
+        // stage j + 1 has landed everywhere and no wavefront reads stage j any more: its slot takes
+        // stage j + 3
+        publish_stage<kOps>(j, KB - 2);
+        next_stage();
+        read_a(st1, 0, nxt);
+        read_b(st1, q ^ 1);
+      } else {
+        read_a(st, i + 1, nxt);
+      }
       v8h a16[4];
-      if (i >= NF) widen_fp8_operand(a, a16);
 #pragma unroll
-      for (int n = 0; n < 4; n++) {
-        const float4 sc = n < 2 ? su : sg;
-        v4f p;
-        if (i >= NF) {
-          v8h b16[4];
-          widen_fp8_operand(B[n], b16);
-          p = mfma_f16_block(a16, b16, v4f{0.f, 0.f, 0.f, 0.f});
-        } else {
-          p = mfma16x16x128(a, B[n], v4f{0.f, 0.f, 0.f, 0.f});
+      for (int h = 0; h < 2; h++) {
+        // (the empty asm keeps this half's MFMAs and the previous m-tile's FMAs in it)
+        asm volatile("" : "+v"(A[cur]), "+v"(p[nxt][2 * h]), "+v"(p[nxt][2 * h + 1]));
+        if (h == 0) {
+          su[cur] = sa[cur] * swu;
+          sg[cur] = sa[cur] * swg;
+          if (i >= NF) widen_fp8_operand(A[cur], a16);
         }
-        acc[i][n][0] += p[0] * sc.x;
-        acc[i][n][1] += p[1] * sc.y;
-        acc[i][n][2] += p[2] * sc.z;
-        acc[i][n][3] += p[3] * sc.w;
+#pragma unroll
+        for (int n = 2 * h; n < 2 * h + 2; n++) {
+          if (i < NF) {
+            p[cur][n] = mfma16x16x128(B[q][n], A[cur], v4f{0.f, 0.f, 0.f, 0.f});
+          } else {
+            v8h b16[4];
+            widen_fp8_operand(B[q][n], b16);
+            p[cur][n] = mfma_f16_block(b16, a16, v4f{0.f, 0.f, 0.f, 0.f});
+          }
+          retire(prev, nxt, n);
+        }
+        if (i < NF) {
+#pragma unroll
+          for (int n = 0; n < 2; n++) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // one MFMA,
+            __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);   // then VALU
+          }
+        }
+        if (i == NT - 1) issue_part(j + 3, ring_lds + slot, h);
+        else issue_part(j + 2, ring_lds + slot2, 2 * (i + 1) + h);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    // stage (j + 2) % 3 was last read at step j - 1, before this step's barrier
-    issue(j + kBgStages - 1);
+    slot = slot1;
+  };
+  int j = 0;
+  for (; j + 2 <= KB; j += 2) {
+    kblock(j, std::integral_constant<int, 0>{});
+    kblock(j + 1, std::integral_constant<int, 1>{});
   }
-  MOEFP8_WAIT_VMCNT(0);
+  auto retire_last = [&](int d) {
+#pragma unroll
+    for (int n = 0; n < 4; n++) retire(NT - 1, d, n);
+  };
+  if (j < KB) {
+    kblock(j, std::integral_constant<int, 0>{});
+    if constexpr (NT > 0) retire_last((NT - 1) & 1);
+  } else {
+    if constexpr (NT > 0) retire_last((2 * NT - 1) & 1);
+  }
+  // every wavefront's DMAs and LDS reads are done: the ring's first stage takes the row maxima
+  publish_stage<0>();
+  float(*amax_s)[kBigRows] = reinterpret_cast<float(*)[kBigRows]>(ring);
   // the workgroup's next unit, claimed now so that the atomic overlaps the epilogue
   if (threadIdx.x == 0) *next_s = grab_unit(pl.queues, n_units);
 
-  // epilogue: C = silu(gate) * up, per-row max over the unit's 128 columns, hi/lo split
-  const int col0 = cb * kBlock + 32 * wn;
-  float c[NT][2][4];
-#pragma unroll
-  for (int i = 0; i < NT; i++)
-#pragma unroll
-    for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) c[i][jn][r] = silu_f32(acc[i][jn + 2][r]) * acc[i][jn][r];
+  // epilogue: C = silu(gate) * up (columns 8 kg .. 8 kg + 7 of the wavefront's 32, for token lr of
+  // each m-tile), per-row max over the unit's 128 columns, hi/lo split
 #pragma unroll
   for (int i = 0; i < NT; i++) {
-    const int t = tile(i);
+    float m = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float m = fmaxf(fabsf(c[i][0][r]), fabsf(c[i][1][r]));
-      m = fmaxf(m, dpp_f32<kDppXor1>(m));
-      m = fmaxf(m, dpp_f32<kDppXor2>(m));
-      m = fmaxf(m, dpp_f32<kDppHalfMirror>(m));
-      m = fmaxf(m, dpp_f32<kDppRowMirror>(m));
-      if (lr == 0) amax_s[wn][16 * t + 4 * kg + r] = m;
-    }
+    for (int n = 0; n < 2; n++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        acc[i][n][r] = silu_f32(acc[i][n + 2][r]) * acc[i][n][r];
+        m = fmaxf(m, fabsf(acc[i][n][r]));
+      }
+    m = fmaxf(m, shfl_xor_f(m, 16));
+    m = fmaxf(m, shfl_xor_f(m, 32));
+    if (kg == 0) amax_s[wn][16 * tile(i) + lr] = m;
   }
   __syncthreads();
+  const int col0 = cb * kBlock + 32 * wn + 8 * kg;
 #pragma unroll
   for (int i = 0; i < NT; i++) {
-    const int t = tile(i);
+    const int R = 16 * tile(i) + lr;
+    if (!rm.valid(R)) continue;
+    const float amax = fmaxf(fmaxf(amax_s[0][R], amax_s[1][R]), fmaxf(amax_s[2][R], amax_s[3][R]));
+    float inv, scale;
+    split_scale(amax, inv, scale);
+    const size_t pr = (size_t)rm.src(R);
+    v8h hi, lo;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int R = 16 * t + 4 * kg + r;
-      if (!rm.valid(R)) continue;
-      const float amax = fmaxf(fmaxf(amax_s[0][R], amax_s[1][R]), fmaxf(amax_s[2][R], amax_s[3][R]));
-      float inv, scale;
-      split_scale(amax, inv, scale);
-      const size_t p = (size_t)rm.src(R);
+    for (int n = 0; n < 2; n++)
 #pragma unroll
-      for (int jn = 0; jn < 2; jn++) store_c(ch, p, I, col0 + 16 * jn + lr, c[i][jn][r], inv);
-      if (wn == 0 && lr == 0) ch.scale[p * NCB + cb] = scale;
-    }
+      for (int r = 0; r < 4; r++) {
+        _Float16 h, l;
+        split_f16(acc[i][n][r], inv, h, l);
+        hi[4 * n + r] = h;
+        lo[4 * n + r] = l;
+      }
+    *reinterpret_cast<v8h*>(ch.hi + pr * I + col0) = hi;
+    *reinterpret_cast<v8h*>(ch.lo16 + pr * I + col0) = lo;
+    if (wn == 0 && kg == 0) ch.scale[pr * NCB + cb] = scale;
   }
 }
 
-// Units (m-block, 128 C columns) over the blocks (128-row class 0/1 blocks, mixed blocks and
-// 32-row exact-product blocks).
+// Units (m-block, 128 C columns) over the blocks (class 0/1 blocks, mixed blocks and 32-row
+// exact-product blocks).
 // One workgroup per CU (its LDS ring), i.e. two wavefronts per SIMD: stated, so that the compiler
 // schedules the K loop for that occupancy instead of squeezing registers for three.
 __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm1_big_kernel(
     Problem pb, Plan pl, CHalf8 ch) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[kBgStages * kBgStage];
-  __shared__ __attribute__((aligned(16))) float2 sw_s[kBigMaxKB];
-  __shared__ float amax_s[4][kBgRows];
-  const int H = pb.H, I = pb.I, KB = H / kBlock, NCB = I / kBlock;
-  // where wavefronts 2..7 put their row-scale DMA (never read)
-  __shared__ __attribute__((aligned(16))) uint32_t dma_sink[64];
-  const uint32_t sink_lds = uniform((int)lds_addr(dma_sink));
   __shared__ int next_s;
+  const int I = pb.I, NCB = I / kBlock;
   const uint32_t ring_lds = uniform((int)lds_addr(ring));
   const int n_units = pl.info[2] * NCB;
   if (threadIdx.x == 0) next_s = first_unit(pl.queues, n_units);
@@ -803,52 +807,45 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     const int4 blk = pl.mblocks[mb];
     const int e = uniform(blk.x), row0 = uniform(blk.y), rows = uniform(blk.z), flags = uniform(blk.w);
     const bool once = uniform(pl.mbgroup[mb].y) == 1;   // the expert's only m-block
-    // the previous unit's readers are done with the ring, amax_s and sw_s, and every thread has
-    // read next_s
-    __syncthreads();
-    // weight scales of the unit: {up, gate} per K-block
-    {
-      const float* su = pb.s13 + ((size_t)e * (2 * I / kBlock) + cb) * KB;
-      const float* sg = su + (size_t)NCB * KB;
-      const int t = threadIdx.x;
-      if (t < KB) sw_s[t] = float2{su[t], sg[t]};
-    }
+    // the previous unit's readers are done with the ring and every thread has read next_s
     __syncthreads();
     const RowMap rm = row_map(row0, rows, flags);
-    const int wm = wave_index() & 1;
-#define MOEFP8_G1_UNIT(NF, NX, TF0, TX0) \
-  gemm1_big_mixed_unit<NF, NX>(pb, pl, ch, ring, ring_lds, sink_lds, sw_s, amax_s, e, rm, cb, TF0, TX0, &next_s, \
-                               n_units)
+    const TileSplit ts = tile_split(rm, flags, wave_index() >> 2);
+    const int nf = uniform(ts.nf), nx = uniform(ts.nx), tf0 = uniform(ts.tf0), tx0 = uniform(ts.tx0);
+#define MOEFP8_G1_UNIT(NF, NX, KA, ONCE) \
+  gemm1_big_unit<NF, NX, KA, ONCE>(pb, pl, ch, ring, ring_lds, e, rm, cb, tf0, tx0, &next_s, n_units)
     if (flags & kFlagMixed) {
-      const TileSplit ts = mixed_split(rm, wm);
-      const int nf = uniform(ts.nf), tf0 = uniform(ts.tf0), tx0 = uniform(ts.tx0);
-      if (ts.nx == 0) {
-        if (nf == 1) MOEFP8_G1_UNIT(1, 0, tf0, 0);
-        else if (nf == 2) MOEFP8_G1_UNIT(2, 0, tf0, 0);
-        else if (nf == 3) MOEFP8_G1_UNIT(3, 0, tf0, 0);
-        else MOEFP8_G1_UNIT(4, 0, tf0, 0);
+      if (nx == 0) {
+        if (nf == 1) MOEFP8_G1_UNIT(1, 0, 2, false);
+        else if (nf == 2) MOEFP8_G1_UNIT(2, 0, 2, false);
+        else if (nf == 3) MOEFP8_G1_UNIT(3, 0, 2, false);
+        else MOEFP8_G1_UNIT(4, 0, 2, false);
       } else {
-        if (nf == 0) MOEFP8_G1_UNIT(0, 1, 0, tx0);
-        else if (nf == 1) MOEFP8_G1_UNIT(1, 1, tf0, tx0);
-        else if (nf == 2) MOEFP8_G1_UNIT(2, 1, tf0, tx0);
-        else MOEFP8_G1_UNIT(3, 1, tf0, tx0);
+        if (nf == 0) MOEFP8_G1_UNIT(0, 1, 2, false);
+        else if (nf == 1) MOEFP8_G1_UNIT(1, 1, 2, false);
+        else if (nf == 2) MOEFP8_G1_UNIT(2, 1, 2, false);
+        else MOEFP8_G1_UNIT(3, 1, 2, false);
       }
+    } else if (flags & kFlagExactProducts) {
+      if (nx) MOEFP8_G1_UNIT(0, 1, 1, false);
+      else MOEFP8_G1_UNIT(0, 0, 1, false);
+    } else if (rows <= 64) {
+      if (once) {
+        if (nf == 0) MOEFP8_G1_UNIT(0, 0, 1, true);
+        else if (nf == 1) MOEFP8_G1_UNIT(1, 0, 1, true);
+        else MOEFP8_G1_UNIT(2, 0, 1, true);
+      } else {
+        if (nf == 0) MOEFP8_G1_UNIT(0, 0, 1, false);
+        else if (nf == 1) MOEFP8_G1_UNIT(1, 0, 1, false);
+        else MOEFP8_G1_UNIT(2, 0, 1, false);
+      }
+    } else if (rows <= 128) {
+      if (nf == 2) MOEFP8_G1_UNIT(2, 0, 2, false);
+      else if (nf == 3) MOEFP8_G1_UNIT(3, 0, 2, false);
+      else MOEFP8_G1_UNIT(4, 0, 2, false);
     } else {
-#define MOEFP8_G1_REG(NT, EXACT) \
-  if (once) gemm1_big_unit<NT, EXACT, true>(pb, pl, ch, ring, ring_lds, sink_lds, sw_s, amax_s, e, row0, rows, cb, \
-                                            &next_s, n_units); \
-  else gemm1_big_unit<NT, EXACT, false>(pb, pl, ch, ring, ring_lds, sink_lds, sw_s, amax_s, e, row0, rows, cb, \
-                                        &next_s, n_units)
-      if (flags & kFlagExactProducts) {
-        MOEFP8_G1_REG(1, true);
-      } else if (rows <= 32) {
-        MOEFP8_G1_REG(1, false);
-      } else if (rows <= 64) {
-        MOEFP8_G1_REG(2, false);
-      } else {
-        MOEFP8_G1_REG(4, false);
-      }
-#undef MOEFP8_G1_REG
+      if (nf == 4) MOEFP8_G1_UNIT(4, 0, 3, false);
+      else MOEFP8_G1_UNIT(5, 0, 3, false);
     }
 #undef MOEFP8_G1_UNIT
     // next_s is written
@@ -1063,10 +1060,10 @@ __global__ __launch_bounds__(kLgThreads, 2) void gemm2_large_kernel(Problem pb, 
 // LDS stage: hi [128 rows][128 B] and lo [128 rows][128 B] (chunks swizzled by slot_key8), W2
 // [256 rows][64 B] (chunk c of row r in slot c ^ bg_key4(r)), 128 row scales of C.
 constexpr int kB2Cols = 256;
-constexpr int kB2Hi = kBgRows * 128;
-constexpr int kB2Lo = kBgRows * 128;
+constexpr int kB2Hi = kGemm2Rows * 128;
+constexpr int kB2Lo = kGemm2Rows * 128;
 constexpr int kB2W = kB2Cols * 64;
-constexpr int kB2Stage = kB2Hi + kB2Lo + kB2W + kBgRows * 4;
+constexpr int kB2Stage = kB2Hi + kB2Lo + kB2W + kGemm2Rows * 4;
 constexpr int kB2Stages = 3;
 
 // 4-slot swizzle of 64-byte rows: chunk c of row r sits in slot c ^ key(r), key linear in the row
@@ -1258,8 +1255,8 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int pass) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[kB2Stages * kB2Stage];
   __shared__ float sw2_s[2 * kBigMaxKB];
-  __shared__ float pw_s[kBgRows];
-  __shared__ int rowp_s[kBgRows];
+  __shared__ float pw_s[kGemm2Rows];
+  __shared__ int rowp_s[kGemm2Rows];
   // the row table's groups: per expert its first GEMM2 row, one- and two-term row counts, first block
   __shared__ int g_off[kEGlobal + 1], g_c1[kEGlobal], g_c2[kEGlobal], g_first[kEGlobal + 1];
   const int H = pb.H, I = pb.I, KB = I / kBlock, HB = H / kBlock, E = pb.E_local;
@@ -1283,7 +1280,7 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     int carry = 0;
     for (int e0 = 0; e0 < E; e0 += kWave) {
       const int ee = e0 + (int)threadIdx.x;
-      const int nb = ee < E ? (g_c1[ee] + kBgRows - 1) / kBgRows + (g_c2[ee] + kBgRows - 1) / kBgRows : 0;
+      const int nb = ee < E ? (g_c1[ee] + kGemm2Rows - 1) / kGemm2Rows + (g_c2[ee] + kGemm2Rows - 1) / kGemm2Rows : 0;
       const int first = carry + wave_exclusive_sum(nb);
       if (ee < E) g_first[ee] = first;
       carry = __builtin_amdgcn_readlane(first + nb, kWave - 1);
@@ -1306,11 +1303,11 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     }
     const int e = uniform(lo), nb = g_first[e + 1] - g_first[e], local = v - g_first[e] * hcn;
     const int hcl = uniform(local / nb), hc = hc0 + hcl, b = local % nb;
-    const int c1 = g_c1[e], b1 = (c1 + kBgRows - 1) / kBgRows;
+    const int c1 = g_c1[e], b1 = (c1 + kGemm2Rows - 1) / kGemm2Rows;
     const bool two = uniform(b >= b1 ? 1 : 0) != 0;
     const int j = two ? b - b1 : b;
-    const int row0 = uniform(g_off[e] + (two ? c1 : 0) + kBgRows * j);
-    const int rows = uniform(min(kBgRows, (two ? g_c2[e] : c1) - kBgRows * j));
+    const int row0 = uniform(g_off[e] + (two ? c1 : 0) + kGemm2Rows * j);
+    const int rows = uniform(min(kGemm2Rows, (two ? g_c2[e] : c1) - kGemm2Rows * j));
     // the previous unit's readers are done with the ring, sw2_s, pw_s and rowp_s, and every thread
     // has read next_s
     __syncthreads();
@@ -1319,7 +1316,7 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     {
       const int t = threadIdx.x;
       if (t < 2 * KB) sw2_s[t] = pb.s2[((size_t)e * HB + 2 * hc + (t & 1)) * KB + (t >> 1)];
-      if (t < kBgRows) {
+      if (t < kGemm2Rows) {
         const int p = clamp_index(pl.g2_pair[row0 + min(t, rows - 1)], pl.pair_rows);
         rowp_s[t] = p;
         pw_s[t] = pl.perm_w[p];
@@ -1476,7 +1473,6 @@ void launch_gemm1_large(const Problem& pb, const Plan& pl, const CHalf8& ch, int
 }
 
 void launch_gemm1_big(const Problem& pb, const Plan& pl, const CHalf8& ch, int max_units, hipStream_t stream) {
-  static_assert(kBigRows == kBgRows, "block height");
   const int cus = num_compute_units();
   const int grid = max_units < cus ? max_units : cus;
   if (grid <= 0) return;

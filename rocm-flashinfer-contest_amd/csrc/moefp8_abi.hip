@@ -118,9 +118,11 @@ static Layout make_layout(int64_t T, int E_local, int H, int I) {
   L.rows_cap = pmax;
   L.nblk = permute_large_blocks(T);
   const int ra = large_rows_a(T, E_local, H, I), rb = large_rows_b(T, E_local, H, I);
-  // blocks per expert (both GEMMs): ceil(class 0+1 rows / ra) + ceil(class 2 rows / rb)
+  // blocks per expert: ceil(class 0+1 rows / ra) + ceil(class 2 rows / rb), or with exact rows folded in
+  // (row_blocks) at most ceil(class 0+1 rows / kMixedRows) + 1: kMixedRows <= ra bounds both
   const int64_t exact_blocks = (pmax + rb - 1) / rb + E_local;
-  L.max_blocks = (pmax + ra - 1) / ra + E_local + exact_blocks;
+  const int64_t rm = ra < kMixedRows ? ra : kMixedRows;
+  L.max_blocks = (pmax + rm - 1) / rm + E_local + exact_blocks;
   L.canon_token = take((size_t)pmax * 4);
   L.bcnt = take((size_t)L.nblk * E_local * 3 * 4);
   L.mblocks = take((size_t)L.max_blocks * 16);
@@ -128,7 +130,7 @@ static Layout make_layout(int64_t T, int E_local, int H, int I) {
   L.two_term = take((size_t)L.max_blocks * 4);
   L.queues = take((size_t)kUnitQueues * kQueueStride * 4);
   // GEMM2's row table (128-row path): its blocks split each expert's rows in two groups
-  L.max_blocks2 = (pmax + kBigRows - 1) / kBigRows + 2 * (int64_t)E_local;
+  L.max_blocks2 = (pmax + kGemm2Rows - 1) / kGemm2Rows + 2 * (int64_t)E_local;
   L.g2_pair = take((size_t)pmax * 4);
   L.g2_ctl = take((size_t)(2 * E_local) * 4);
   L.xrow = take((size_t)E_local * 4);

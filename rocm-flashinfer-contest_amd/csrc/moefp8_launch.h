@@ -143,8 +143,9 @@ struct LargePermArgs {
   int* queues;          // [kUnitQueues * kQueueStride] unit queues of the grouped GEMMs, zeroed here
   int* g2_ctl;          // [2 E_local] GEMM2 row-table counters, zeroed here (NULL: none)
   int* xrow;            // [E_local] first exact-product (class 2) row of each local expert
-  int mixed;            // fold <= 32 exact-product rows into the expert's last class 0/1 block
-  int rows_a;           // block height over an expert's class 0 and 1 rows
+  int mixed;            // fold <= 32 exact-product rows into the expert's last class 0/1 block, and cut an
+                        // expert's rows into blocks of about equal height
+  int rows_a;           // largest block height over an expert's class 0 and 1 rows (a multiple of 32)
   int rows_b;           // block height over its class 2 (exact-product) rows
 };
 void launch_permute_large(const LargePermArgs& args, hipStream_t stream);
@@ -161,9 +162,11 @@ int large_grid();
 // GEMM1 over its blocks [0, info[2]), 16 * mt rows per block
 void launch_gemm1_large(const Problem& pb, const Plan& pl, const CHalf8& ch, int mt, int max_units,
                         hipStream_t stream);
-// GEMM1 over the whole table (kBigRows-row class 0/1 blocks, 32-row exact-product blocks), one
-// workgroup per CU
-constexpr int kBigRows = 128;
+// GEMM1 over the whole table (class 0/1 blocks of up to kBigRows rows, those with exact-product rows
+// folded in of up to kMixedRows, 32-row exact-product blocks), one workgroup per CU
+constexpr int kBigRows = 160;
+constexpr int kMixedRows = 128;
+constexpr int kGemm2Rows = 128;   // GEMM2's largest block
 constexpr int kBigMaxKB = 64;   // H <= 8192
 void launch_gemm1_big(const Problem& pb, const Plan& pl, const CHalf8& ch, int max_units, hipStream_t stream);
 // GEMM2's precision flags (Plan::two_term) of the blocks [0, info[2]) from GEMM1's output

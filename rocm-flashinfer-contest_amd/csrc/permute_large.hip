@@ -37,11 +37,28 @@ __device__ __forceinline__ int class_flags(int c) {
 
 // Does an expert with n01 class 0/1 rows and n2 exact-product rows fold the latter into its last
 // class 0/1 block (a mixed block: the exact rows take the block's last ceil(n2 / 16) m-tiles)?
-// Only with 128-row blocks, at most 32 exact rows and room for them.
 __device__ __forceinline__ bool folds_exact(const LargePermArgs& a, int n01, int n2) {
-  if (!a.mixed || n2 < 1 || n2 > 32 || n01 < 1) return false;
-  const int last = n01 - (n01 - 1) / a.rows_a * a.rows_a;
-  return last <= a.rows_a - 16 * ((n2 + 15) / 16);
+  return a.mixed && n2 >= 1 && n2 <= 32 && n01 >= 1;
+}
+
+// The blocks over an expert's class 0/1 rows, in steps of 32 rows: n of them, the first r of q + 1 steps and
+// the others of q (the last ends with the rows).  Without `mixed`, blocks of rows_a rows.  With it the fewest
+// blocks of at most rows_a rows, of about equal height: 260 rows as 160 + 100 and not 128 + 128 + 4, since
+// a block streams its expert's whole weight slice however short it is.  Folded exact rows count as one step of
+// the last block, whose height then stays within kMixedRows (q <= 4; q >= 2, so it keeps class 0/1 rows too).
+struct RowBlocks {
+  int n, q, r;
+  __device__ __forceinline__ int first(int j) const { return 32 * (j * q + min(j, r)); }
+};
+__device__ __forceinline__ RowBlocks row_blocks(const LargePermArgs& a, int n01, int n2) {
+  const int per = a.rows_a / 32;
+  if (!a.mixed) return RowBlocks{(n01 + a.rows_a - 1) / a.rows_a, per, 0};
+  const bool fold = folds_exact(a, n01, n2);
+  const int steps = (n01 + 31) / 32 + (fold ? 1 : 0);
+  int n = (steps + per - 1) / per;
+  if (fold && steps == n * per) n++;
+  const int q = n > 0 ? steps / n : 0;
+  return RowBlocks{n, q, steps - n * q};
 }
 
 // A token's 8 slots (local expert or -1, routing weight) and squared norm, and one thread's share
@@ -159,7 +176,7 @@ __device__ __forceinline__ int upper_bound(const int* v, int n, int x) {
 }
 
 // Expert offsets, 16-row m-tile offsets and m-block offsets, expert by expert, from the bucket
-// totals (one wavefront): blocks of rows_a rows over an expert's class 0 and 1 rows (two-term C in
+// totals (one wavefront): blocks over an expert's class 0 and 1 rows (row_blocks; two-term C in
 // the blocks that hold class 1 rows), then blocks of rows_b rows over its class 2 rows, or those
 // folded into its last class 0/1 block (folds_exact: 27 of 107 blocks at T = 8192 held <= 32 exact
 // rows each, a quarter of the GEMMs' weight streams for 5% of the rows).  The grouped GEMMs run
@@ -175,7 +192,7 @@ __device__ void expert_offsets(const LargePermArgs& a, const int* tot, int* eoff
     const int n0 = e < E ? tot[kClasses * e] : 0, n1 = e < E ? tot[kClasses * e + 1] : 0;
     const int n2 = e < E ? tot[kClasses * e + 2] : 0, n = n0 + n1 + n2;
     const int mt = (n + 15) / 16;
-    const int ba = (n0 + n1 + a.rows_a - 1) / a.rows_a;
+    const int ba = row_blocks(a, n0 + n1, n2).n;
     const int bx = folds_exact(a, n0 + n1, n2) ? 0 : (n2 + a.rows_b - 1) / a.rows_b;
     const int b1 = ba + bx;
     const int pn = wave_exclusive_sum(n), pmt = wave_exclusive_sum(mt);
@@ -221,9 +238,10 @@ __device__ void write_mblocks(const LargePermArgs& a, const int* tot, const int*
   for (int g = threadIdx.x; g < eb1[E]; g += blockDim.x) {
     const int e = upper_bound(eb1, E + 1, g) - 1, j = g - eb1[e];
     const int c0 = tot[kClasses * e], c01 = c0 + tot[kClasses * e + 1], n = eoff[e + 1] - eoff[e];
-    const int ba = (c01 + a.rows_a - 1) / a.rows_a;
+    const RowBlocks rb = row_blocks(a, c01, n - c01);
+    const int ba = rb.n;
     if (j < ba) {
-      const int r0 = j * a.rows_a, rows = min(a.rows_a, c01 - r0);
+      const int r0 = rb.first(j), rows = min(rb.first(j + 1), c01) - r0;
       int flags = r0 + rows > c0 ? class_flags(1) : 0;
       if (j == ba - 1 && folds_exact(a, c01, n - c01)) flags |= kFlagMixed | ((n - c01) << kMixedShift);
       a.mblocks[g] = int4{e, eoff[e] + r0, rows, flags};

@@ -1,0 +1,84 @@
+"""Rows per expert at the edges of the prefill GEMMs' blocks and m-tiles, against the CPU oracle.
+
+Each token is routed to exactly one chosen local expert (its other seven picks lie in other groups), so
+an expert's row count, and how many of its rows take exact products, are what the case says."""
+import pytest
+import torch
+
+import moe_oracle as O
+import moe_fp8
+from moe_fp8 import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+ATOL, RTOL = 1e-2, 2e-2      # the operator's bar
+E_LOCAL = 4
+
+
+def case_inputs(counts, exact, T, H, I, seed):
+    """counts[e] rows for local expert e, the first exact[e] of them large (exact products); tokens past
+    them have no local expert.  Tokens of the experts are interleaved."""
+    g = torch.Generator().manual_seed(seed)
+    owner = torch.full((T,), -1)
+    order = torch.randperm(T, generator=g)
+    big, at = torch.zeros(T, dtype=torch.bool), 0
+    for e, n in enumerate(counts):
+        owner[order[at:at + n]] = e
+        big[order[at:at + exact[e]]] = True
+        at += n
+    logits = torch.full((T, 256), -8.0) + 0.1 * torch.randn(T, 256, generator=g)
+    for base in (32, 33, 64, 65, 96, 97, 98, 99):          # eight remote picks in groups 1, 2, 3
+        logits[:, base] = 2.0 + 0.1 * torch.randn(T, generator=g)
+    local = owner >= 0
+    logits[torch.nonzero(local).squeeze(1), owner[local]] = 4.0
+    hidden = torch.randn(T, H, generator=g)
+    hidden[big] *= 60.0
+    hs, hss = W.quantize_rows_1x128(hidden)
+    return logits, torch.zeros(256, dtype=torch.bfloat16), hs, hss
+
+
+def check(counts, exact, T, H, I, seed):
+    act = case_inputs(counts, exact, T, H, I, seed)
+    weights = W.make_weights(E_LOCAL, H, I, device="cpu", seed=91)
+    args = (*act, *weights, 0, W.RSF)
+    dbg = {}
+    out = moe_fp8.run(*(a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args), debug=dbg)
+    torch.cuda.synchronize()
+    assert dbg["expert_offsets"].cpu().diff().tolist() == list(counts)
+    ref32, _ = O.moe_forward(*args)
+    err = (out.float().cpu() - ref32).abs()
+    bad = int((err > ATOL + RTOL * ref32.abs()).sum())
+    assert bad == 0, f"{bad} elements outside the bar, max abs err {float(err.max()):.3e}"
+    none = torch.ones(T, dtype=torch.bool)
+    off = dbg["expert_offsets"].cpu()
+    none[dbg["permuted_tokens"].cpu()[:off[-1]].long()] = False
+    assert torch.all(out.cpu()[none] == 0)
+
+
+@pytest.mark.parametrize("T", [0, 1100])           # just the rows (at least 140 tokens), and past 1024 tokens
+@pytest.mark.parametrize("counts", [(1, 15, 16, 17), (31, 32, 33, 0), (63, 64, 65, 2), (95, 96, 97, 3),
+                                    (127, 128, 129, 4), (159, 160, 161, 5), (191, 193, 0, 224), (255, 256, 257, 33),
+                                    (319, 320, 321, 48)])
+def test_rows_per_expert(counts, T):
+    T = max(T, sum(counts), 140)
+    print(f"[rows] {counts} T={T}", flush=True)
+    check(counts, (0,) * E_LOCAL, T, 512, 256, seed=sum(counts))
+
+
+@pytest.mark.parametrize("T", [0, 1100])
+@pytest.mark.parametrize("counts,exact", [((1, 2, 16, 17), (1, 1, 16, 16)), ((33, 48, 49, 64), (1, 16, 17, 32)),
+                                          ((97, 128, 129, 160), (1, 17, 32, 32)), ((161, 193, 225, 300), (33, 32, 16, 40)),
+                                          ((290, 320, 40, 35), (1, 32, 40, 3))])
+def test_exact_rows_per_expert(counts, exact, T):
+    """1 to 32 exact rows fold into an expert's last block, more get blocks of their own."""
+    T = max(T, sum(counts), 140)
+    print(f"[exact rows] {counts} exact {exact} T={T}", flush=True)
+    check(counts, exact, T, 512, 256, seed=7 + sum(counts))
+
+
+@pytest.mark.parametrize("H,I", [(256, 128), (768, 384), (256, 1152), (2048, 640)])
+def test_odd_shapes(H, I):
+    """One, three, nine and five K-blocks in GEMM2; two to sixteen in GEMM1."""
+    print(f"[shapes] H={H} I={I}", flush=True)
+    check((5, 40, 70, 130), (0, 3, 0, 33), 300, H, I, seed=H + I)
