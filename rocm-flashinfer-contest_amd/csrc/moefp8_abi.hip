@@ -466,6 +466,8 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
   pa.mixed = big ? 1 : 0;   // the 128-row GEMMs run mixed blocks
   pa.rows_a = large_rows_a(T, E_local, H, I);
   pa.rows_b = large_rows_b(T, E_local, H, I);
+  pa.units = I / kBlock;
+  pa.slots = num_compute_units();
   pl.canon_token = pa.canon_token;
   pl.mblocks = pa.mblocks;
   pl.mbgroup = pa.mbgroup;

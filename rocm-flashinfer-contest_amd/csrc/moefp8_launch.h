@@ -147,6 +147,7 @@ struct LargePermArgs {
                         // expert's rows into blocks of about equal height
   int rows_a;           // largest block height over an expert's class 0 and 1 rows (a multiple of 32)
   int rows_b;           // block height over its class 2 (exact-product) rows
+  int units, slots;     // with `mixed`: GEMM1's units per block and its workgroups
 };
 void launch_permute_large(const LargePermArgs& args, hipStream_t stream);
 int permute_large_blocks(int64_t T);
@@ -166,6 +167,7 @@ void launch_gemm1_large(const Problem& pb, const Plan& pl, const CHalf8& ch, int
 // folded in of up to kMixedRows, 32-row exact-product blocks), one workgroup per CU
 constexpr int kBigRows = 160;
 constexpr int kMixedRows = 128;
+constexpr int kBigRowsLow = 128;   // the lower of the two largest heights that the permutation chooses from
 constexpr int kGemm2Rows = 128;   // GEMM2's largest block
 constexpr int kBigMaxKB = 64;   // H <= 8192
 void launch_gemm1_big(const Problem& pb, const Plan& pl, const CHalf8& ch, int max_units, hipStream_t stream);
