@@ -19,21 +19,21 @@ namespace moefp8 {
 // Largest T served by the weight-streaming kernels.
 constexpr int64_t kDecodeMaxT = 64;
 
-// Large-T m-blocks.  From T = 128 the class 0/1 rows of an expert go in 128-row blocks for the
-// LDS-staged 128-row GEMMs and its exact-product rows in 32-row blocks (or folded into the last
-// class 0/1 block): even with a few rows per expert these stream each weight slice once per
-// block and took 253 / 249 / 277 / 311 µs at T = 128 / 256 / 512 / 1024 against 262 / 252 / 288
-// / 389 µs for the 4-wave kernels below.  Those (blocks of 16 * large_mt(T) rows) remain for
-// 64 < T < 128 and for shapes the 128-row kernels do not take.
+// Large-T m-blocks: the class 0/1 rows of an expert go in blocks of up to kBigRows rows for the LDS-staged
+// GEMM1 and its exact-product rows in 32-row blocks (or folded into the last class 0/1 block), from T = 65 on:
+// even with a few rows per expert this streams each weight slice once per block, with GEMM2's streaming kernel
+// 207 / 218 / 241 / 240 us at T = 65 / 80 / 100 / 127 against 246 / 258 / 278 / 276 us for the 4-wave
+// kernels below.  Those (blocks of 16 * large_mt(T) rows) remain for shapes the staged kernels do not take.
+// kBigT is where moefp8_path's MOEFP8_PATH_ROWS128 begins (per-pair precision of C in GEMM2).
 constexpr int64_t kBigT = 128;
 constexpr int kExactRows = 32;
-// The 128-row kernels address their DMA sources with 32-bit per-lane byte offsets from a
+// The staged kernels address their DMA sources with 32-bit per-lane byte offsets from a
 // wave-uniform base: hidden rows (token x H, GEMM1) and C rows (pair x 2I, GEMM2).  Shapes whose
 // offsets could pass 2^31 (T x H) or 2^32 (Pmax x 2I, Pmax = T x min(8, E_local)) take the 4-wave
 // kernels, which form 64-bit addresses.
 bool large_big(int64_t T, int E_local, int H, int I) {
   const int64_t pmax = T * (E_local < kTopK ? E_local : kTopK);
-  return T >= kBigT && H / kBlock <= kBigMaxKB && I / kBlock <= kBigMaxKB && H % 256 == 0 &&
+  return T > kDecodeMaxT && H / kBlock <= kBigMaxKB && I / kBlock <= kBigMaxKB && H % 256 == 0 &&
          T * H < ((int64_t)1 << 31) && pmax * 2 * I < ((int64_t)1 << 32);
 }
 int large_mt(int64_t T) { return T / 32 >= 48 ? 4 : 2; }
@@ -48,7 +48,7 @@ int large_mt(int64_t T) { return T / 32 >= 48 ? 4 : 2; }
 constexpr size_t kOutRowsBudget = (size_t)1 << 30;
 int64_t output_rows(int64_t T, int E_local, int H, int I) {
   const int64_t pmax = T * (E_local < kTopK ? E_local : kTopK);
-  if (T <= kDecodeMaxT || !large_big(T, E_local, H, I) || (size_t)pmax * H * 4 <= kOutRowsBudget) return pmax;
+  if (!large_big(T, E_local, H, I) || (size_t)pmax * H * 4 <= kOutRowsBudget) return pmax;
   // rows of the first (larger) half of the columns for every pair: ceil(pmax * half / H) full rows
   const int64_t half = (H / 256 + 1) / 2 * 256;
   return (pmax * half + H - 1) / H;
@@ -260,8 +260,9 @@ int moefp8_path(int64_t num_tokens, int32_t num_local_experts, int32_t hidden_si
   const int rc = check_sizes(num_tokens, num_local_experts, hidden_size, intermediate_size);
   if (rc) return rc;
   if (num_tokens <= kDecodeMaxT) return MOEFP8_PATH_SMALL_T;
-  return large_big(num_tokens, num_local_experts, hidden_size, intermediate_size) ? MOEFP8_PATH_ROWS128
-                                                                                    : MOEFP8_PATH_GROUPED;
+  return num_tokens >= kBigT && large_big(num_tokens, num_local_experts, hidden_size, intermediate_size)
+             ? MOEFP8_PATH_ROWS128
+             : MOEFP8_PATH_GROUPED;
 }
 
 int moefp8_output_passes(int64_t num_tokens, int32_t num_local_experts, int32_t hidden_size,
@@ -365,6 +366,7 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
   pl.g2_pair = nullptr;
   pl.g2_ctl = nullptr;
   pl.xrow = nullptr;
+  pl.tok_a2 = nullptr;
   pl.shared = a->shared_output;
   pl.shared_dt = a->shared_dtype;
   pl.out_f32 = a->output_f32;
@@ -478,6 +480,7 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
   pa.g2_ctl = big ? pl.g2_ctl : nullptr;
   pa.xrow = reinterpret_cast<int*>(ws + L.xrow);
   pl.xrow = pa.xrow;
+  pl.tok_a2 = tok_a2;
   CHalf8 ch;
   ch.hi = reinterpret_cast<_Float16*>(ws + L.c_hi);
   ch.lo16 = reinterpret_cast<_Float16*>(ws + L.c_lo16);
@@ -497,7 +500,10 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
   mark(3);
   // GEMM2's precision from the C that GEMM1 wrote (the activation stage): per pair, with GEMM2's
   // own row table, on the 128-row path; per m-block otherwise
-  if (big) {
+  const bool stream2 = big && T <= kStreamT && L.o_rows >= L.pmax;
+  if (stream2) {
+    // (the stream kernel decides per block, from the scales of the block that it reads)
+  } else if (big) {
     launch_g2_plan(pb, pl, ch, (int)L.pmax, s);
   } else {
     launch_c_flags(pl, ch, I, (int)L.max_blocks, s);
@@ -510,7 +516,8 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
     // (its two empty launches cost ~7 us per call, measured)
     const int passes = L.o_rows >= L.pmax ? 1 : 2;
     for (int pass = 0; pass < 2; pass++) {
-      if (pass < passes) launch_gemm2_big(pb, pl, ch, obuf, (int)(L.max_blocks2 * (H / 256)), (int)L.o_rows, pass, s);
+      if (stream2 && pass == 0) launch_gemm2_stream(pb, pl, ch, obuf, T < kBigT, s);
+      else if (pass < passes) launch_gemm2_big(pb, pl, ch, obuf, (int)(L.max_blocks2 * (H / 256)), (int)L.o_rows, pass, s);
       mark(5 + 2 * pass);
       if (pass < passes) launch_combine_pass(pl, obuf, a->output, (int)T, H, (int)L.o_rows, pass, s);
       mark(6 + 2 * pass);

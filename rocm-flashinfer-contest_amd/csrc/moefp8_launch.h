@@ -85,6 +85,7 @@ struct Plan {
   int* g2_ctl;                // [2 E_local] one- / two-term row counts per expert (zeroed by the
                               // permutation)
   const int* xrow;            // [E_local] first exact-product row of each local expert (permutation)
+  const float* tok_a2;        // [T] squared norm of each dequantised hidden row (routing)
 };
 
 struct Problem {
@@ -195,6 +196,12 @@ __device__ __forceinline__ OutPass out_pass(int P, int H, int o_rows, int pass, 
 // pass `pass` (out_pass)
 void launch_gemm2_big(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, int max_units, int o_rows,
                       int pass, hipStream_t stream);
+
+// GEMM2 for T <= kStreamT on the same C and O (one pass over the columns): C resident in LDS, W2 streamed.
+// With `by_estimate` a block also takes both terms of C for a row of magnitude class 1.
+constexpr int kStreamT = 512;
+void launch_gemm2_stream(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, bool by_estimate,
+                         hipStream_t stream);
 
 void launch_combine(const Plan& pl, const float* obuf, void* out, int T, int H, hipStream_t stream);
 // The combine of output pass `pass` (out_pass) of the 128-row path.

@@ -77,8 +77,10 @@ def test_exact_rows_per_expert(counts, exact, T):
     check(counts, exact, T, 512, 256, seed=7 + sum(counts))
 
 
+@pytest.mark.parametrize("counts,exact", [((5, 40, 70, 130), (0, 3, 0, 33)), ((64, 128, 16, 17), (0, 64, 16, 0))])
 @pytest.mark.parametrize("H,I", [(256, 128), (768, 384), (256, 1152), (2048, 640)])
-def test_odd_shapes(H, I):
-    """One, three, nine and five K-blocks in GEMM2; two to sixteen in GEMM1."""
-    print(f"[shapes] H={H} I={I}", flush=True)
-    check((5, 40, 70, 130), (0, 3, 0, 33), 300, H, I, seed=H + I)
+def test_odd_shapes(H, I, counts, exact):
+    """One, three, nine and five K-blocks in GEMM2 (nine: more than one or both terms of a tall block's C hold
+    in LDS at once); two to sixteen in GEMM1."""
+    print(f"[shapes] H={H} I={I} {counts}", flush=True)
+    check(counts, exact, 300, H, I, seed=H + I)
