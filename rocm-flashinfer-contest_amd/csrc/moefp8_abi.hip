@@ -26,7 +26,6 @@ constexpr int64_t kDecodeMaxT = 64;
 // kernels below.  Those (blocks of 16 * large_mt(T) rows) remain for shapes the staged kernels do not take.
 // kBigT is where moefp8_path's MOEFP8_PATH_ROWS128 begins (per-pair precision of C in GEMM2).
 constexpr int64_t kBigT = 128;
-constexpr int kExactRows = 32;
 // The staged kernels address their DMA sources with 32-bit per-lane byte offsets from a
 // wave-uniform base: hidden rows (token x H, GEMM1) and C rows (pair x 2I, GEMM2).  Shapes whose
 // offsets could pass 2^31 (T x H) or 2^32 (Pmax x 2I, Pmax = T x min(8, E_local)) take the 4-wave

@@ -188,15 +188,19 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
   return (readlane_f32(v, 0) + readlane_f32(v, 16)) + (readlane_f32(v, 32) + readlane_f32(v, 48));
 }
 
-// Exclusive prefix sum over the wavefront (Hillis-Steele on shuffles).
+// Exclusive prefix sum over the wavefront, through DPP (six dependent adds; as shuffles, six LDS round trips).
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ int dpp_or_zero(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xF, false);
+}
 __device__ __forceinline__ int wave_exclusive_sum(int v) {
-  const int lane = lane_id();
   int x = v;
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const int y = __shfl_up(x, off, kWave);
-    if (lane >= off) x += y;
-  }
+  x += dpp_or_zero<0x111, 0xF>(x);   // row_shr:1, 2, 4, 8: inside rows of 16 lanes
+  x += dpp_or_zero<0x112, 0xF>(x);
+  x += dpp_or_zero<0x114, 0xF>(x);
+  x += dpp_or_zero<0x118, 0xF>(x);
+  x += dpp_or_zero<0x142, 0xA>(x);   // row_bcast:15 into rows 1 and 3
+  x += dpp_or_zero<0x143, 0xC>(x);   // row_bcast:31 into rows 2 and 3
   return x - v;
 }
 

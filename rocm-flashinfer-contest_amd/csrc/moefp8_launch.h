@@ -168,6 +168,7 @@ void launch_gemm1_large(const Problem& pb, const Plan& pl, const CHalf8& ch, int
 // folded in of up to kMixedRows, 32-row exact-product blocks), one workgroup per CU
 constexpr int kBigRows = 160;
 constexpr int kMixedRows = 128;
+constexpr int kExactRows = 32;     // exact-product rows of a block of their own
 constexpr int kBigRowsLow = 128;   // the lower of the two largest heights that the permutation chooses from
 constexpr int kGemm2Rows = 128;   // GEMM2's largest block
 constexpr int kBigMaxKB = 64;   // H <= 8192

@@ -1,11 +1,11 @@
 // Permutation of the (token, local expert) pairs for T > 64, in two launches over blocks of
-// 256 tokens (one token per thread):
+// 256 tokens (one token per thread), or up to kSelfBlocks blocks in the second alone:
 //
 //   count  per block, the number of pairs in each bucket (local expert, magnitude class)
-//   place  per block, from all blocks' counts (staged in LDS): every bucket's total and this
-//          block's prefix of it, hence the bucket and expert offsets; each pair's rank inside its
-//          bucket in token order then gives its row, the rank inside its expert alone its
-//          canonical row.  Block 0 also writes the offsets and the m-block table of the grouped
+//   place  per block, from all blocks' counts (staged in LDS; up to kSelfBlocks blocks count for
+//          themselves): every bucket's total and this block's prefix of it, hence the bucket and
+//          expert offsets; each pair's rank inside its bucket in token order then gives its row,
+//          the rank inside its expert alone its canonical row.  Block 0 also writes the offsets and the m-block table of the grouped
 //          GEMMs.  (A one-workgroup scan launch between the two took 5-7 us plus a launch
 //          boundary at T = 1024-8192; every block redoing the sums it needs costs it one round of
 //          loads.)
@@ -41,6 +41,11 @@ __device__ __forceinline__ bool folds_exact(const LargePermArgs& a, int n01, int
   return a.mixed && n2 >= 1 && n2 <= 32 && n01 >= 1;
 }
 
+// Blocks over n2 exact-product rows that are not folded.
+__device__ __forceinline__ int exact_blocks(const LargePermArgs& a, int n2) {
+  return a.mixed ? (n2 + kExactRows - 1) / kExactRows : (n2 + a.rows_b - 1) / a.rows_b;
+}
+
 // The blocks over an expert's class 0/1 rows, in steps of 32 rows: n of them, the first r of q + 1 steps and
 // the others of q (the last ends with the rows).  Without `mixed`, blocks of rows_a rows.  With it the fewest
 // blocks of at most rows_a rows, of about equal height: 260 rows as 160 + 100 and not 160 + 96 + 4, since
@@ -51,12 +56,12 @@ struct RowBlocks {
   __device__ __forceinline__ int first(int j) const { return 32 * (j * q + min(j, r)); }
 };
 __device__ __forceinline__ RowBlocks row_blocks(const LargePermArgs& a, int rows_a, int n01, int n2) {
-  const int per = rows_a / 32;
-  if (!a.mixed) return RowBlocks{(n01 + rows_a - 1) / rows_a, per, 0};
-  const bool fold = folds_exact(a, n01, n2);
+  if (!a.mixed) return RowBlocks{(n01 + rows_a - 1) / rows_a, rows_a / 32, 0};
+  const bool fold = folds_exact(a, n01, n2), high = rows_a == kBigRows;
   const int steps = (n01 + 31) / 32 + (fold ? 1 : 0);
-  int n = (steps + per - 1) / per;
-  if (fold && steps == n * per) n++;
+  constexpr int kHigh = kBigRows / 32, kLow = kBigRowsLow / 32;   // (divisions by constants)
+  int n = high ? (steps + kHigh - 1) / kHigh : (steps + kLow - 1) / kLow;
+  if (fold && steps == n * (high ? kHigh : kLow)) n++;
   const int q = n > 0 ? steps / n : 0;
   return RowBlocks{n, q, steps - n * q};
 }
@@ -164,6 +169,37 @@ __device__ void bucket_sums(const LargePermArgs& a, int me, int* tot, int* pre, 
   __syncthreads();
 }
 
+// The same by counting every token's buckets here, for at most kSelfBlocks blocks: a token more per thread instead
+// of a launch and its round trip through memory.  The two launches are latency (15-18 us for some KB): with one,
+// and the prefix sums on DPP, 11-15 us; calls at T = 100 242.6 -> 239.8 us, 200 252.9 -> 250.1, 500 269.5 -> 267.0.
+// With 4 blocks a call at T = 600 measured 295.6 us against 297.0 by two launches, at 768 302.2 and 303.4, at 1024
+// 318.3 and 317.6, within what runs differ, and T = 500 (a pass more) 269.0 instead of 267.9: the line stays at 2.
+// All threads of the block (es is published by its first barrier); ends with a barrier.
+constexpr int kSelfBlocks = 2;
+__device__ void bucket_counts(const LargePermArgs& a, int me, int* tot, int* pre, const float* es) {
+  const int E3 = a.E_local * kClasses, tid = threadIdx.x;
+  for (int i = tid; i < E3; i += kBlkTokens) {
+    tot[i] = 0;
+    pre[i] = 0;
+  }
+  TokenSlots ts[kSelfBlocks];
+#pragma unroll
+  for (int q = 0; q < kSelfBlocks; q++) load_token_slots(a, q * kBlkTokens + tid, ts[q]);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kSelfBlocks; q++) {
+    if (q * kBlkTokens + tid >= a.T) continue;
+#pragma unroll
+    for (int k = 0; k < kTopK; k++) {
+      const int b = slot_bucket(a, ts[q], k, es);
+      if (b < 0) continue;
+      atomicAdd(&tot[b], 1);
+      if (q < me) atomicAdd(&pre[b], 1);
+    }
+  }
+  __syncthreads();
+}
+
 // First index i in [0, n) with v[i] > x (v ascending).
 __device__ __forceinline__ int upper_bound(const int* v, int n, int x) {
   int lo = 0, hi = n;
@@ -185,23 +221,24 @@ __device__ __forceinline__ int upper_bound(const int* v, int n, int x) {
 // An expert's blocks are consecutive, so the units that stream its weights run close together in
 // time and share them through L2.  With `write`, also the path's global tables.
 //
-// Returns the largest block height.  With `mixed` it is kBigRows, or kBigRowsLow where that takes GEMM1 no more
-// rounds of units over its workgroups: the same number of rounds of shorter units.  GEMM1's calls at zipf routing:
+// Returns the largest block height (meaningful with `write` alone: only the tables depend on it).  With `mixed` it
+// is kBigRows, or kBigRowsLow where that takes GEMM1 no more rounds of units over its workgroups: the same number
+// of rounds of shorter units.  GEMM1's calls at zipf routing:
 // T = 1000 234 us at 160, 225 at 128 (as many rounds); T = 1500 256 and 285 us (one round more at 128).
 __device__ int expert_offsets(const LargePermArgs& a, const int* tot, int* eoff, int* emt, int* eb1, bool write) {
   const int E = a.E_local, lane = lane_id();
   int rows_a = a.rows_a;
-  if (a.mixed) {
+  if (a.mixed && write) {
     int high = 0, low = 0, rest = 0;
     for (int e = lane; e < E; e += kWave) {
       const int n01 = tot[kClasses * e] + tot[kClasses * e + 1], n2 = tot[kClasses * e + 2];
       high += row_blocks(a, kBigRows, n01, n2).n;
       low += row_blocks(a, kBigRowsLow, n01, n2).n;
-      rest += folds_exact(a, n01, n2) ? 0 : (n2 + a.rows_b - 1) / a.rows_b;
+      rest += folds_exact(a, n01, n2) ? 0 : exact_blocks(a, n2);
     }
     // (counts below 2^24: exact in fp32)
-    const int uh = (int)(wave_sum_f32((float)high) + wave_sum_f32((float)rest)) * a.units;
-    const int ul = (int)(wave_sum_f32((float)low) + wave_sum_f32((float)rest)) * a.units;
+    const int uh = (int)wave_sum_f32((float)(high + rest)) * a.units;
+    const int ul = (int)wave_sum_f32((float)(low + rest)) * a.units;
     if ((ul + a.slots - 1) / a.slots <= (uh + a.slots - 1) / a.slots) rows_a = kBigRowsLow;
   }
   int carry = 0, carry_mt = 0, carry_1 = 0, carry_act = 0;
@@ -211,7 +248,7 @@ __device__ int expert_offsets(const LargePermArgs& a, const int* tot, int* eoff,
     const int n2 = e < E ? tot[kClasses * e + 2] : 0, n = n0 + n1 + n2;
     const int mt = (n + 15) / 16;
     const int ba = row_blocks(a, rows_a, n0 + n1, n2).n;
-    const int bx = folds_exact(a, n0 + n1, n2) ? 0 : (n2 + a.rows_b - 1) / a.rows_b;
+    const int bx = folds_exact(a, n0 + n1, n2) ? 0 : exact_blocks(a, n2);
     const int b1 = ba + bx;
     const int pn = wave_exclusive_sum(n), pmt = wave_exclusive_sum(mt);
     const int p1 = wave_exclusive_sum(b1);
@@ -288,6 +325,8 @@ __device__ __forceinline__ void wave_key_ranks(const int (&key)[kTopK], int (&ra
   for (int k = 0; k < kTopK; k++) rank[k] = key[k] >= 0 ? (int)__popcll(masks[key[k]] & (me - 1)) : 0;
 }
 
+// kSelf: no count launch has run (at most kSelfBlocks blocks).
+template <bool kSelf>
 __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a) {
   // per wavefront and key, the lanes holding it: buckets (expert x class) and experts
   __shared__ unsigned long long bmask[kBlkWaves][kEGlobal * kClasses];
@@ -296,7 +335,7 @@ __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a)
   // bucket totals and this block's prefix of them; expert, m-tile and m-block offsets
   __shared__ int tot[kEGlobal * kClasses], pre[kEGlobal * kClasses];
   __shared__ int eoff[kEGlobal + 1], emt[kEGlobal + 1], eb1[kEGlobal + 1];
-  __shared__ int stage[kPlaceLdsInts];
+  __shared__ int stage[kSelf ? 1 : kPlaceLdsInts];
   __shared__ int rows_a;   // largest block height
   const int E = a.E_local, E3 = E * kClasses, tid = threadIdx.x, wave = tid >> 6;
   const int t = blockIdx.x * kBlkTokens + tid;
@@ -306,7 +345,8 @@ __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a)
   for (int i = tid; i < kBlkWaves * E3; i += kBlkTokens) bmask[i / E3][i % E3] = 0ull;
   for (int i = tid; i < kBlkWaves * E; i += kBlkTokens) emask[i / E][i % E] = 0ull;
   stage_esig(a, ts, es);
-  bucket_sums(a, blockIdx.x, tot, pre, stage);
+  if constexpr (kSelf) bucket_counts(a, blockIdx.x, tot, pre, es);
+  else bucket_sums(a, blockIdx.x, tot, pre, stage);
   const bool first = blockIdx.x == 0;
   if (wave == 0) {
     const int r = expert_offsets(a, tot, eoff, emt, eb1, first);
@@ -367,8 +407,12 @@ __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a)
 
 void launch_permute_large(const LargePermArgs& args, hipStream_t stream) {
   if (args.nblk <= 0) return;
+  if (args.nblk <= kSelfBlocks) {
+    hipLaunchKernelGGL(perm_place_kernel<true>, dim3(args.nblk), dim3(kBlkTokens), 0, stream, args);
+    return;
+  }
   hipLaunchKernelGGL(perm_count_kernel, dim3(args.nblk), dim3(kBlkTokens), 0, stream, args);
-  hipLaunchKernelGGL(perm_place_kernel, dim3(args.nblk), dim3(kBlkTokens), 0, stream, args);
+  hipLaunchKernelGGL(perm_place_kernel<false>, dim3(args.nblk), dim3(kBlkTokens), 0, stream, args);
 }
 
 int permute_large_blocks(int64_t T) { return (int)((T + kBlkTokens - 1) / kBlkTokens); }
