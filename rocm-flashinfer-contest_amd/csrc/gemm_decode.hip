@@ -24,8 +24,7 @@
 //             exact products of C's f16 hi term (2^-11 relative) and W2 widened to f16;
 //             the last unit to finish a 64-column block then sums each token's pair rows
 //             and splits over those columns into the bf16 output   (main.py:241-243).
-// M-tiles flagged for exact products (GEMM1) or for both f16 terms of C (GEMM2) take a
-// simpler per-wavefront path.
+// M-tiles flagged for exact products in GEMM1 take a simpler per-wavefront path.
 #include "decode_plan.h"
 #include "moefp8_device.h"
 #include "moefp8_launch.h"
@@ -53,12 +52,6 @@ __device__ __forceinline__ v8i load_v8i(const uint8_t* p) {
   const v4i* q = reinterpret_cast<const v4i*>(p);
   const v4i x = q[0], y = q[1];
   return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
-__device__ __forceinline__ void load_v8h4(const _Float16* p, v8h (&y)[4]) {
-  const v8h* q = reinterpret_cast<const v8h*>(p);
-#pragma unroll
-  for (int i = 0; i < 4; i++) y[i] = q[i];
 }
 
 // Unit u -> (m-tile g, K-split s, column block cb of 4 groups), column block fastest.
@@ -545,13 +538,11 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
     const bool two = ((uniform(mt.w) & kFlagTwoTermC) | uniform(measured)) != 0;
     const int kb0 = du.s * KB / S, n = (du.s + 1) * KB / S - kb0;
     const int cg = du.cb * kDecBlockWaves + wave;
-    const uint8_t* bp = pb.w2 + ((size_t)e * H + cg * 16 + lr) * I + (size_t)kb0 * kBlock + kg * 32;
     const float* swp = pb.s2 + ((size_t)e * HB + (cg * 16) / kBlock) * KB + kb0;
-    const int prow = row0 + (lr < M ? lr : 0);
     v4f acc = {0.f, 0.f, 0.f, 0.f};
 
     if (!two && M <= kPreRows && n <= kPre2MaxKB) {
-      const float swv = swp[min(lane, n - 1)];
+      float swv = swp[min(lane, n - 1)];
       // weights as whole lines, transposed per wavefront through LDS (as in GEMM1)
       const int wr = lane >> 3, wc = lane & 7;
       const uint8_t* wsrc = pb.w2 + ((size_t)e * H + cg * 16 + wr) * I + (size_t)kb0 * kBlock + wc * 16;
@@ -584,7 +575,12 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
           v[q] = *reinterpret_cast<const v4i*>(ch.hi + (size_t)(row0 + r) * I + (size_t)kb0 * kBlock + c * 8);
         }
         const int si = min((int)threadIdx.x, M * n - 1), sr = si / n, sj = si - sr * n;
-        const float sv = ch.scale[(size_t)(row0 + sr) * KB + kb0 + sj];
+        float sv = ch.scale[(size_t)(row0 + sr) * KB + kb0 + sj];
+        // (pinned: sunk below the stores' branches or into the loop, the loads are waited for one by one, the
+        // last with all weights in flight: run() 82.5 against 81.4 us at T = 16)
+#pragma unroll
+        for (int q = 0; q < kPer; q++) asm volatile("" : "+v"(v[q]));
+        asm volatile("" : "+v"(sv));
 #pragma unroll
         for (int q = 0; q < kPer; q++) {
           const int i = threadIdx.x + q * 64 * kDecBlockWaves;
@@ -593,6 +589,7 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
         }
         if ((int)threadIdx.x < M * n) sh.pre.sa[sj][sr] = sv;
         __syncthreads();
+        asm volatile("" : "+v"(swv));
       }
       // rows >= M read row M - 1 (real data, results discarded)
       const uint8_t* arow = sh.pre.a + min(lr, M - 1) * kPre2RowBytes + kg * 64;
@@ -627,14 +624,24 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
       for (int d = 0; d < kDecDepth - 1; d++)
         if (j + d < n) step(d, j + d);
       __syncthreads();
-    } else if (!two) {
+    } else {
       constexpr int kStepDepth2 = 2;   // (register budget shared with the staged path)
-      // carriers: wave q loads rows 4q .. 4q + 3 of C's hi term as whole lines (lane l: row
-      // 4q + l/16, 16-byte chunk l%16) and publishes them to the stage; wave 0's lanes < 16 the
-      // scale of row lane (all lanes load it: no loads under a branch)
-      const int ar = 4 * wave + (lane >> 4);
-      const _Float16* asrc = ch.hi + (size_t)(row0 + (ar < M ? ar : 0)) * I + (size_t)kb0 * kBlock + (lane & 15) * 8;
-      const float* ssrc = ch.scale + (size_t)prow * KB + kb0;
+      // Both terms of C (M of any size): with M <= 8 the lo term is operand rows 8 .. 8 + M - 1, in the
+      // same matrix products as the hi rows; with more rows a step of its own after each hi step
+      // (`alt`: step i is K-block i / 2), on the same weights again.  An unpipelined loop over
+      // MFMA-layout loads had both terms as operands: GEMM2 122 us at T = 64 with lognormal rows against
+      // 72 us for one term, now 71; calls at T = 16 / 48 / 64 66 / 199 / 255 -> 61 / 151 / 193 us.
+      // (Up to 2 such rows on the staged path above, as 4 operand rows: no faster.)
+      const bool rows8 = two && M <= 8;
+      const int alt = two && !rows8 ? 1 : 0, steps = n << alt;
+      // carriers: wave q loads rows 4q .. 4q + 3 as whole lines (lane l: row 4q + l/16, 16-byte
+      // chunk l%16) and publishes them to the stage; wave 0's lanes < 16 the scale of row lane (all
+      // lanes load it: no loads under a branch)
+      const int ar = 4 * wave + (lane >> 4), ac = rows8 ? ar & 7 : ar, sc = rows8 ? lr & 7 : lr;
+      const _Float16* asrc = (rows8 && ar >= 8 ? ch.lo : ch.hi) + (size_t)(row0 + (ac < M ? ac : 0)) * I +
+                             (size_t)kb0 * kBlock + (lane & 15) * 8;
+      const ptrdiff_t lo_step = alt ? ch.lo - ch.hi : 0;
+      const float* ssrc = ch.scale + (size_t)(row0 + (sc < M ? sc : 0)) * KB + kb0;
       const float swv = swp[min(lane, n - 1)];
       // weights as whole lines with the non-temporal hint, transposed per wavefront through its LDS
       // buffer tb as on the staged path (MFMA-layout loads instead: 184.8 against 173.9 us per call
@@ -650,10 +657,10 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
       v4i AR[kStepDepth2];
       float SR[kStepDepth2];
       auto load = [&](int d, int j) {
-        const int jj = min(j, n - 1);
+        const int i = min(j, steps - 1), jj = i >> alt;
         B0[d] = load_w_line(wsrc + (size_t)jj * kBlock);
         B1[d] = load_w_line(wsrc + (size_t)jj * kBlock + (size_t)8 * I);
-        AR[d] = *reinterpret_cast<const v4i*>(asrc + (size_t)jj * kBlock);
+        AR[d] = *reinterpret_cast<const v4i*>(asrc + (size_t)jj * kBlock + (i & alt ? lo_step : 0));
         SR[d] = ssrc[jj];
       };
       auto step = [&](int d, int j) {
@@ -673,7 +680,7 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
         int rb = lr * (2 * kBlock) + ((4 * kg) ^ slot_key16(lr)) * 16;
         asm volatile("" : "+v"(rb));
         const float4 sa = *reinterpret_cast<const float4*>(st.sa + 4 * kg);
-        const float sw = readlane_f32(swv, j);
+        const float sw = readlane_f32(swv, j >> alt);
         // one 32-K piece at a time (C's hi chunk, the W2 chunk widened exactly, their MFMA), in
         // the order of widen_fp8_operand + mfma_f16_block: all four pieces widened at once
         // spilled 4 VGPRs
@@ -698,7 +705,7 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
 #pragma unroll
       for (int d = 0; d < kStepDepth2; d++) load(d, d);
       int j = 0;
-      for (; j + kStepDepth2 <= n; j += kStepDepth2) {
+      for (; j + kStepDepth2 <= steps; j += kStepDepth2) {
 #pragma unroll
         for (int d = 0; d < kStepDepth2; d++) {
           step(d, j + d);
@@ -708,32 +715,11 @@ __global__ __launch_bounds__(64 * kDecBlockWaves, kDec2BlocksPerCU) void gemm2_d
       }
 #pragma unroll
       for (int d = 0; d < kStepDepth2 - 1; d++)
-        if (j + d < n) step(d, j + d);
+        if (j + d < steps) step(d, j + d);
       __syncthreads();
-    } else {
-      const _Float16* hp = ch.hi + (size_t)prow * I + (size_t)kb0 * kBlock + kg * 32;
-      const _Float16* lp = ch.lo + (size_t)prow * I + (size_t)kb0 * kBlock + kg * 32;
-      const float* sp[4];
+      if (rows8) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int dr = 4 * kg + r;
-        sp[r] = ch.scale + (size_t)(row0 + (dr < M ? dr : 0)) * KB + kb0;
-      }
-      for (int j = 0; j < n; j++) {
-        const v8i b = load_v8i(bp + (size_t)j * kBlock);
-        v8h ah[4], al[4];
-        load_v8h4(hp + (size_t)j * kBlock, ah);
-        load_v8h4(lp + (size_t)j * kBlock, al);
-        float sa[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) sa[r] = sp[r][j];
-        const float sw = swp[j];
-        v8h b16[4];
-        widen_fp8_operand(b, b16);
-        v4f p = mfma_f16_block(ah, b16, v4f{0.f, 0.f, 0.f, 0.f});
-        p = mfma_f16_block(al, b16, p);
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[r] += p[r] * (sa[r] * sw);
+        for (int r = 0; r < 4; r++) acc[r] += __shfl_xor(acc[r], 32, kWave);   // row 8 + i onto row i
       }
     }
 #pragma unroll

@@ -1,4 +1,4 @@
-"""Rows per expert at the edges of the prefill GEMMs' blocks and m-tiles, against the CPU oracle.
+"""Rows per expert at the edges of the GEMMs' blocks and m-tiles, against the CPU oracle.
 
 Each token is routed to exactly one chosen local expert (its other seven picks lie in other groups), so
 an expert's row count, and how many of its rows take exact products, are what the case says."""
@@ -84,3 +84,25 @@ def test_odd_shapes(H, I, counts, exact):
     in LDS at once); two to sixteen in GEMM1."""
     print(f"[shapes] H={H} I={I} {counts}", flush=True)
     check(counts, exact, 300, H, I, seed=H + I)
+
+
+@pytest.mark.parametrize("big", [0, 1])
+@pytest.mark.parametrize("H,I", [(512, 256), (256, 128), (768, 640), (2048, 1152)])
+@pytest.mark.parametrize("counts", [(1, 2, 3, 4), (5, 7, 8, 9), (15, 16, 17, 8), (24, 25, 1, 0), (0, 0, 64, 0)])
+def test_two_terms_small_batch(counts, H, I, big):
+    """Up to 64 tokens, every m-tile on both terms of C: 1 to 8 rows (hi and lo rows of one tile) and 9 to 16
+    (steps of their own).  C in one f16 term errs by 2^-11 / sqrt(3) = 2.8e-4 of each element (rms over its binade
+    and over the sum about 1.5e-4 of a row), in two by 2^-22, below the fp32 sums' own 1e-6 to 1e-5."""
+    print(f"[two terms] {counts} H={H} I={I} big={big}", flush=True)
+    T = min(64, sum(counts) + 3)
+    act = case_inputs(counts, counts if big else (0,) * E_LOCAL, T, H, I, seed=3 + sum(counts) + I)
+    logits, bias, hs, hss = act
+    weights = list(W.make_weights(E_LOCAL, H, I, device="cpu", seed=91))
+    if not big:
+        hss = hss * 16.0
+    args = (logits, bias, hs, hss, *weights, 0, W.RSF)
+    out = moe_fp8.run(*(a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args), output_dtype=torch.float32)
+    torch.cuda.synchronize()
+    ref32, _ = O.moe_forward(*args)
+    err = float((out.cpu() - ref32).norm() / ref32.norm())
+    assert err < 5e-5, f"relative error {err:.2e}"
