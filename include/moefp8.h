@@ -132,9 +132,10 @@ int moefp8_workspace_size(int64_t num_tokens, int32_t num_local_experts, int32_t
 
 /* Kernel family moefp8_run uses for these sizes (host only, no device needed; no counterpart in
  * the reference, whose run() always loops over experts in Python, main.py:218-241):
- * MOEFP8_PATH_SMALL_T (T <= 64: weight-streaming GEMMs), MOEFP8_PATH_GROUPED (64 < T < 128, and
- * shapes outside the LDS-staged GEMMs' range) or MOEFP8_PATH_ROWS128 (LDS-staged grouped GEMMs with
- * per-pair precision of C, from T = 128), or a negative status. */
+ * MOEFP8_PATH_SMALL_T (T <= 64: weight-streaming GEMMs), MOEFP8_PATH_GROUPED (64 < T < 128, where
+ * the precision of C follows the magnitude estimate too, and shapes outside the LDS-staged GEMMs' range) or
+ * MOEFP8_PATH_ROWS128 (the LDS-staged GEMMs, precision of C from C itself, from T = 128), or a negative
+ * status. */
 #define MOEFP8_PATH_SMALL_T 0
 #define MOEFP8_PATH_GROUPED 1
 #define MOEFP8_PATH_ROWS128 2

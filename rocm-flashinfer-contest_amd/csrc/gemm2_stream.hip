@@ -38,7 +38,6 @@ constexpr int kStShortDepth = 4;                  // the same where a pass holds
 constexpr int kStCBytes = 128 * 1024;             // C in LDS
 constexpr int kStPad = 16;                        // bytes between LDS rows of C, so that an MFMA operand read
                                                   // (16 rows, 64 bytes per lane group) has no bank conflicts
-constexpr int kStMaxKB = 64;                      // I <= 8192
 
 // K-blocks of `planes` = m-tiles x terms planes of 16 rows that fit LDS, a multiple of the ring depth.
 __host__ __device__ constexpr int stream_depth(int planes) { return planes <= 4 ? kStDepth : kStShortDepth; }

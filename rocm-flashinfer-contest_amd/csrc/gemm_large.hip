@@ -1,5 +1,7 @@
-// Grouped expert GEMMs for T > 64 (prefill): LDS-staged activations, per-wavefront
-// weight streams.
+// Grouped expert GEMMs for T > 64 (prefill).  Three families: the LDS-staged ones with both operands in LDS
+// (GEMM1 of every call in their range, GEMM2 past kStreamT tokens; their own headers below), gemm2_stream.hip for
+// GEMM2 up to there, and for the shapes outside that range (large_big) the 4-wave ones described here:
+// LDS-staged activations, per-wavefront weight streams.
 //
 // A workgroup of 4 wavefronts owns one unit = (m-block of BM = 16*MT rows of one expert,
 // block of 128 output columns).  Each wavefront streams its own 32 or 64 weight rows
@@ -19,7 +21,7 @@
 //        products: f16 MFMA on widened operands), SwiGLU in the epilogue (main.py:229-233),
 //        and C written as hi = f16(C/s), s = max|C row block| / 448 per 128 cols, and
 //        lo = f16(C/s - hi) (22 significant bits together).
-// flags  per m-block, whether GEMM2 needs both terms of C (needs_two_terms on each row's max |C|
+// flags  per m-block (4-wave kernels), whether GEMM2 needs both terms of C (needs_two_terms on each row's max |C|
 //        per 128 columns, from the scales GEMM1 wrote).
 // GEMM2  O = C W2_e^T (main.py:234-238): C's hi term on the f16 MFMA against W2 widened
 //        to f16 (exact products, 2^-11 relative input error); m-blocks flagged by GEMM1 add

@@ -440,7 +440,7 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
     mark(8);
     return finish(a, L, topk_ids, topk_w, pl, s);
   }
-  // large T: routing, permutation (3 launches), GEMM1 (+SwiGLU, C split), GEMM2, combine
+  // large T: routing, permutation (1 or 2 launches), GEMM1 (+SwiGLU, C split), GEMM2, combine
   LargePermArgs pa = {};
   pa.topk_ids = topk_ids;
   pa.topk_w = topk_w;
@@ -464,7 +464,7 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
   pa.mbgroup = reinterpret_cast<int2*>(ws + L.mbgroup);
   pa.queues = reinterpret_cast<int*>(ws + L.queues);
   const bool big = large_big(T, E_local, H, I);
-  pa.mixed = big ? 1 : 0;   // the 128-row GEMMs run mixed blocks
+  pa.mixed = big ? 1 : 0;   // the LDS-staged GEMMs run mixed blocks
   pa.rows_a = large_rows_a(T, E_local, H, I);
   pa.rows_b = large_rows_b(T, E_local, H, I);
   pa.units = I / kBlock;
@@ -497,8 +497,8 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
     launch_gemm1_large(pb, pl, ch, large_mt(T), (int)(L.max_blocks * (I / kBlock)), s);
   }
   mark(3);
-  // GEMM2's precision from the C that GEMM1 wrote (the activation stage): per pair, with GEMM2's
-  // own row table, on the 128-row path; per m-block otherwise
+  // GEMM2's precision from the C that GEMM1 wrote (the activation stage): per pair, with GEMM2's own row
+  // table, for the LDS-staged kernel; by the stream kernel itself; per m-block for the 4-wave ones
   const bool stream2 = big && T <= kStreamT && L.o_rows >= L.pmax;
   if (stream2) {
     // (the stream kernel decides per block, from the scales of the block that it reads)

@@ -71,8 +71,9 @@ __device__ __forceinline__ void split_f16(float x, float inv, _Float16& hi, _Flo
 // the measured rms ~7x).  Used before GEMM1, where only the inputs are known: pairs above
 // kPreciseRms take GEMM1's exact-product path (the fp8 MFMA's adder error is relative to
 // sum |a w|, which this estimate tracks), and pairs above kOneTermRms are grouped together inside
-// their expert and take two terms of C in GEMM2 (kFlagTwoTermC) on the small-T and grouped paths
-// (the 128-row path decides each row's terms from its measured C alone, g2_plan_kernel).
+// their expert and take two terms of C in GEMM2 (kFlagTwoTermC) below 128 tokens and on the
+// 4-wave kernels (from 128 tokens the LDS-staged path decides from the measured C alone: per row in
+// g2_plan_kernel, per block in gemm2_stream_kernel).
 constexpr float kPreciseRms = 96.0f;
 constexpr float kOneTermRms = 8.0f;
 constexpr uint8_t kFlagExactProducts = 1;
@@ -310,11 +311,6 @@ __device__ __forceinline__ void dma_lds4(const void* g, uint32_t lds_uniform) {
 // The same with a wave-uniform 64-bit base in SGPRs and a 32-bit per-lane byte offset.
 __device__ __forceinline__ void dma_lds16_s(uint32_t voff, const void* sbase, uint32_t lds_uniform) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase),
-               "s"(lds_uniform) : "memory", "m0");
-}
-// The same with the non-temporal hint (streamed through L2), for lines read once per call.
-__device__ __forceinline__ void dma_lds16_s_nt(uint32_t voff, const void* sbase, uint32_t lds_uniform) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(voff), "s"(sbase),
                "s"(lds_uniform) : "memory", "m0");
 }
 __device__ __forceinline__ void dma_lds4_s(uint32_t voff, const void* sbase, uint32_t lds_uniform) {

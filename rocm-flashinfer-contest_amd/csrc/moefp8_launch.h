@@ -79,7 +79,7 @@ struct Plan {
   int out_f32;                // output in fp32 (the sum before its bf16 rounding) instead of bf16
   int pair_rows;              // pair rows the workspace holds (perm_token, C, O): pair indices read
                               // from the tables are clamped below it where they become addresses
-  // 128-row path, GEMM2's own row table (built by the g2 plan launch from the C GEMM1 wrote): per
+  // LDS-staged GEMM2, its own row table (built by the g2 plan launch from the C GEMM1 wrote): per
   // expert its one-term rows, then its two-term rows (GEMM2 takes them in blocks of up to 128)
   const int* g2_pair;         // [Pmax] GEMM2 row -> pair row
   int* g2_ctl;                // [2 E_local] one- / two-term row counts per expert (zeroed by the
@@ -154,7 +154,7 @@ void launch_permute_large(const LargePermArgs& args, hipStream_t stream);
 int permute_large_blocks(int64_t T);
 
 // C between the large-T GEMMs: hi = f16(C/s), lo16 = f16(C/s - hi), s = max |C| / 448 per
-// (pair, 128 columns).  GEMM2 reads lo16 only in m-blocks flagged two_term.
+// (pair, 128 columns).  GEMM2 reads lo16 only in blocks of two-term rows.
 struct CHalf8 {
   _Float16* hi;     // [Pmax][I]
   _Float16* lo16;   // [Pmax][I]
@@ -178,7 +178,7 @@ void launch_c_flags(const Plan& pl, const CHalf8& ch, int I, int max_blocks, hip
 // GEMM2 over the blocks [0, info[2]), taken 16 * mt rows at a time
 void launch_gemm2_large(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, int mt, int max_units,
                         hipStream_t stream);
-// GEMM2's row table for the 128-row path (Plan::g2_*): every pair whose C needs both f16 terms
+// The LDS-staged GEMM2's row table (Plan::g2_*): every pair whose C needs both f16 terms
 // (its magnitude class, or needs_two_terms on the C scales GEMM1 wrote) goes to its expert's
 // two-term blocks, the others to its one-term blocks.  Pmax bounds the launch's pair rows.
 void launch_g2_plan(const Problem& pb, const Plan& pl, const CHalf8& ch, int pmax, hipStream_t stream);
@@ -205,7 +205,7 @@ void launch_gemm2_stream(const Problem& pb, const Plan& pl, const CHalf8& ch, fl
                          hipStream_t stream);
 
 void launch_combine(const Plan& pl, const float* obuf, void* out, int T, int H, hipStream_t stream);
-// The combine of output pass `pass` (out_pass) of the 128-row path.
+// The combine of output pass `pass` (out_pass).
 void launch_combine_pass(const Plan& pl, const float* obuf, void* out, int T, int H, int o_rows, int pass,
                          hipStream_t stream);
 
