@@ -86,6 +86,14 @@ def test_odd_shapes(H, I, counts, exact):
     check(counts, exact, 300, H, I, seed=H + I)
 
 
+@pytest.mark.parametrize("T", [65, 255, 256, 257, 511, 512, 513, 769])
+def test_token_block_edges(T):
+    """The permutation's 256-token blocks: one, two (counted by the placing launch itself) and three or four."""
+    print(f"[token blocks] T={T}", flush=True)
+    counts = (T // 3, T // 4, 5, T - T // 3 - T // 4 - 6)
+    check(counts, (T // 9, 0, 1, 3), T, 512, 256, seed=T)
+
+
 @pytest.mark.parametrize("big", [0, 1])
 @pytest.mark.parametrize("H,I", [(512, 256), (256, 128), (768, 640), (2048, 1152)])
 @pytest.mark.parametrize("counts", [(1, 2, 3, 4), (5, 7, 8, 9), (15, 16, 17, 8), (24, 25, 1, 0), (0, 0, 64, 0)])
