@@ -828,26 +828,38 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
         else if (nf == 2) MOEFP8_G1_UNIT(2, 1, 2, false);
         else MOEFP8_G1_UNIT(3, 1, 2, false);
       }
-    } else if (flags & kFlagExactProducts) {
-      if (nx) MOEFP8_G1_UNIT(0, 1, 1, false);
-      else MOEFP8_G1_UNIT(0, 0, 1, false);
-    } else if (rows <= 64) {
-      if (once) {
-        if (nf == 0) MOEFP8_G1_UNIT(0, 0, 1, true);
-        else if (nf == 1) MOEFP8_G1_UNIT(1, 0, 1, true);
-        else MOEFP8_G1_UNIT(2, 0, 1, true);
-      } else {
-        if (nf == 0) MOEFP8_G1_UNIT(0, 0, 1, false);
-        else if (nf == 1) MOEFP8_G1_UNIT(1, 0, 1, false);
-        else MOEFP8_G1_UNIT(2, 0, 1, false);
-      }
-    } else if (rows <= 128) {
-      if (nf == 2) MOEFP8_G1_UNIT(2, 0, 2, false);
-      else if (nf == 3) MOEFP8_G1_UNIT(3, 0, 2, false);
-      else MOEFP8_G1_UNIT(4, 0, 2, false);
     } else {
-      if (nf == 4) MOEFP8_G1_UNIT(4, 0, 3, false);
-      else MOEFP8_G1_UNIT(5, 0, 3, false);
+#define MOEFP8_G1_REG(NF, NX, KA) \
+  if (once) MOEFP8_G1_UNIT(NF, NX, KA, true); \
+  else MOEFP8_G1_UNIT(NF, NX, KA, false)
+      if (flags & kFlagExactProducts) {
+        if (nx) {
+          MOEFP8_G1_REG(0, 1, 1);
+        } else {
+          MOEFP8_G1_REG(0, 0, 1);
+        }
+      } else if (rows <= 64) {
+        if (nf == 0) {
+          MOEFP8_G1_REG(0, 0, 1);
+        } else if (nf == 1) {
+          MOEFP8_G1_REG(1, 0, 1);
+        } else {
+          MOEFP8_G1_REG(2, 0, 1);
+        }
+      } else if (rows <= 128) {
+        if (nf == 2) {
+          MOEFP8_G1_REG(2, 0, 2);
+        } else if (nf == 3) {
+          MOEFP8_G1_REG(3, 0, 2);
+        } else {
+          MOEFP8_G1_REG(4, 0, 2);
+        }
+      } else if (nf == 4) {
+        MOEFP8_G1_REG(4, 0, 3);
+      } else {
+        MOEFP8_G1_REG(5, 0, 3);
+      }
+#undef MOEFP8_G1_REG
     }
 #undef MOEFP8_G1_UNIT
     // next_s is written
