@@ -536,9 +536,10 @@ __device__ __forceinline__ int mask_less(int x, int y) {
 // products (the f16 MFMA on operands widened exactly).  KA: activation DMAs per wavefront and stage (8
 // rows each, 64 rows per step of KA over the 8 wavefronts).  kOnce: the block is its expert's only one, so
 // each weight line is read once per call, by one DMA instruction (8 lanes x 16 B), and its DMAs carry
-// the non-temporal hint: 5% less GEMM1 time at 1024 tokens (about one block per expert), measured.
-// Experts with several blocks keep ordinary DMAs, which let the blocks share the weights through L2
-// (the hint on every block cost 20% at 8192 tokens, measured).
+// the non-temporal hint: 5% less GEMM1 time at 1024 tokens (about one block per expert), and 179 / 188 /
+// 247 us instead of 199 / 214 / 275 at T = 2048 / 3000 / 4096 (blocks of 65 to 160 rows).  Experts with several
+// blocks keep ordinary DMAs, which let the blocks share the weights through L2 (the hint on every block cost
+// 20% at 8192 tokens, measured).
 template <int NF, int NX, int KA, bool kOnce>
 __device__ __forceinline__ void gemm1_big_unit(const Problem& pb, const Plan& pl, const CHalf8& ch, uint8_t* ring,
                                                uint32_t ring_lds, int e, const RowMap& rm, int cb, int tf0, int tx0,
@@ -572,7 +573,6 @@ __device__ __forceinline__ void gemm1_big_unit(const Problem& pb, const Plan& pl
     boff[q] = (uint32_t)(cb * kBlock + bg_wrow(R, I)) * (uint32_t)H + (uint32_t)((dslot ^ slot_key8(R)) * 16);
   }
   const int sgrp = kBgWaves - 1 - wave;
-  // (the stage holds kBigRows scales: the last group is cut to those)
   // (the stage holds kBigRows scales: the last group is cut to those)
   const int s_lo = mask_less(sgrp, KA) & mask_less(64 * sgrp, rm.xrows ? kMixedRows : rm.rows);
   const int s_hi = s_lo & mask_less(64 * sgrp + 32, kBigRows);
@@ -727,20 +727,14 @@ __device__ __forceinline__ void gemm1_big_unit(const Problem& pb, const Plan& pl
     }
     slot = slot1;
   };
-  int j = 0;
-  for (; j + 2 <= KB; j += 2) {
+  // (KB is even: the staged GEMMs take H % 256 == 0 alone)
+  for (int j = 0; j < KB; j += 2) {
     kblock(j, std::integral_constant<int, 0>{});
     kblock(j + 1, std::integral_constant<int, 1>{});
   }
-  auto retire_last = [&](int d) {
+  if constexpr (NT > 0) {
 #pragma unroll
-    for (int n = 0; n < 4; n++) retire(NT - 1, d, n);
-  };
-  if (j < KB) {
-    kblock(j, std::integral_constant<int, 0>{});
-    if constexpr (NT > 0) retire_last((NT - 1) & 1);
-  } else {
-    if constexpr (NT > 0) retire_last((2 * NT - 1) & 1);
+    for (int n = 0; n < 4; n++) retire(NT - 1, (2 * NT - 1) & 1, n);
   }
   // every wavefront's DMAs and LDS reads are done: the ring's first stage takes the row maxima
   publish_stage<0>();
@@ -1059,13 +1053,12 @@ __global__ __launch_bounds__(kLgThreads, 2) void gemm2_large_kernel(Problem pb, 
 }
 
 // ------------------------------------------------------------------------------ GEMM2, 128-row m-blocks
-// For the 128-row blocks.  A workgroup of 8 wavefronts (one per CU, two per SIMD) owns one unit =
-// (m-block, 256 output columns) and stages C's hi term (f16), in blocks GEMM1 flagged also its lo
-// term (f16), and the W2 rows by DMA through a 3-stage LDS ring, 64 K per stage.  Wavefront
-// (wm, wn) = (w % 2, w / 2) computes rows 64 wm .. +63 x output columns 64 wn .. +63 on the f16
-// MFMA 16x16x32 (W2 widened to f16 exactly; the lo term's products chained onto the hi ones).
-// The block's rows come through its row map (a mixed block keeps its exact-product rows in its
-// last m-tiles; GEMM2 treats them like the others).
+// For blocks of up to 128 rows of its own row table (g2_plan_kernel: per expert the rows of one-term C, then
+// those of two-term C).  A workgroup of 8 wavefronts (one per CU, two per SIMD) owns one unit = (block, 256
+// output columns) and stages C's hi term (f16), in two-term blocks also its lo term (f16), and the W2 rows by
+// DMA through a 3-stage LDS ring, 64 K per stage.  Wavefront (wm, wn) = (w % 2, w / 2) computes rows 64 wm ..
+// +63 (32 or 16 of them in blocks of at most 64 or 32 rows) x output columns 64 wn .. +63 on the f16 MFMA
+// 16x16x32 (W2 widened to f16 exactly; the lo term's products chained onto the hi ones).
 //
 // Within a 64-K stage, lane group kg of an MFMA operand holds k = 16 kg + 8 t + (0..7) for the
 // two 32-K MFMAs t = 0, 1 (the same order for both operands): its W2 bytes are one 16-byte
