@@ -16,6 +16,28 @@ ATOL, RTOL = 1e-2, 2e-2      # the operator's bar
 E_LOCAL = 4
 
 
+def cdiv(a, b):
+    return -(-a // b)
+
+
+def compute_units():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+def gemm1_height(counts, exact, I, slots):
+    """The largest block height of the staged GEMM1: 160 rows where that saves a round of units, else 128."""
+    rounds = {}
+    for height in (160, 128):
+        blocks = 0
+        for n, n2 in zip(counts, exact):
+            n01, fold = n - n2, 1 <= n2 <= 32 and n > n2
+            steps = cdiv(n01, 32) + fold
+            k = cdiv(steps, height // 32)
+            blocks += k + (fold and steps == k * (height // 32)) + (0 if fold else cdiv(n2, 32))
+        rounds[height] = cdiv(blocks * (I // 128), slots)
+    return 128 if rounds[128] <= rounds[160] else 160
+
+
 def case_inputs(counts, exact, T, H, I, seed):
     """counts[e] rows for local expert e, the first exact[e] of them large (exact products); tokens past
     them have no local expert.  Tokens of the experts are interleaved."""
@@ -40,7 +62,7 @@ def case_inputs(counts, exact, T, H, I, seed):
 
 def check(counts, exact, T, H, I, seed):
     act = case_inputs(counts, exact, T, H, I, seed)
-    weights = W.make_weights(E_LOCAL, H, I, device="cpu", seed=91)
+    weights = W.make_weights(len(counts), H, I, device="cpu", seed=91)
     args = (*act, *weights, 0, W.RSF)
     dbg = {}
     out = moe_fp8.run(*(a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args), debug=dbg)
@@ -92,6 +114,19 @@ def test_token_block_edges(T):
     print(f"[token blocks] T={T}", flush=True)
     counts = (T // 3, T // 4, 5, T - T // 3 - T // 4 - 6)
     check(counts, (T // 9, 0, 1, 3), T, 512, 256, seed=T)
+
+
+@pytest.mark.parametrize("counts,exact", [((129, 144, 145, 159, 160), (0,) * 5), ((128, 131, 133, 160, 190), (33, 40, 33, 64, 33)),
+                                          ((112, 113, 129, 129, 160), (16, 17, 1, 32, 40)),
+                                          ((33, 97, 160, 270, 320), (1, 32, 0, 17, 0))])
+def test_blocks_of_160_rows(counts, exact):
+    """32 experts of eight GEMM1 units per block: a second round of units if any expert took two blocks.  Class 0/1
+    rows up to 160 in one block, beside exact-product blocks (more than 32 exact rows) and mixed ones (their step of
+    32 rows makes the fifth of an expert's steps a second block)."""
+    counts, exact = (counts * 7)[:32], (exact * 7)[:32]
+    print(f"[160 rows] {counts[:5]} exact {exact[:5]}", flush=True)
+    assert gemm1_height(counts, exact, 1024, compute_units()) == 160
+    check(counts, exact, sum(counts), 256, 1024, seed=sum(counts) + sum(exact))
 
 
 @pytest.mark.parametrize("big", [0, 1])
