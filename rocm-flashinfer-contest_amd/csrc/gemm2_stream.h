@@ -2,16 +2,16 @@
 //
 // O = C W2_e^T (main.py:234-238) with at most a few dozen rows per expert is the time it takes to read W2
 // once.  A plain DMA stream of the 32 experts' W2 (470 MB, this kernel's order, non-temporal) takes 71 us;
-// the LDS-staged kernel of gemm_large.hip, which meets at a barrier every 64 K and drains its pipeline at
-// each of its 3-4 units per CU, takes 108 / 115 / 120 us at T = 128 / 333 / 512 (with the row
-// table's launch, 7 us, before it), this one 83 / 88 / 100 us; with log-normal tokens, many of whose blocks take
-// two terms, 166 against 100 us at T = 250 and 172 against 121 at T = 512.  Past kStreamT = 512 the blocks of hot
-// experts need several passes over K, each restaging 128 KB of C: at zipf routing calls of T = 400 / 512 take 182 /
-// 205 us against 188 / 207, and would take 230 against 217 at T = 700.  Here
+// the LDS-staged units of gemm_large.hip, which meet at a barrier every 64 K and drain their pipeline at
+// each of their 3-4 units per CU, take 108 / 115 / 120 us at T = 128 / 333 / 512, these ones 83 / 88 / 100 us; with
+// log-normal tokens, many of whose blocks take two terms, 166 against 100 us at T = 250 and 172 against 121 at T = 512.
 //
-// * a workgroup (8 wavefronts, one per CU) takes an equal, contiguous share of all (block, 128 output columns)
-//   units, block by block, so that it meets one or two blocks in all and every CU the same work to within
-//   one of about seven units;
+// With many rows per expert the staged units are the better ones: past 32 rows a block's C does not fit LDS over all of
+// K, past 64 W2 is streamed again.  What decides is how the pairs fall on the experts, which only the device
+// knows: gemm2_short_kernel runs either (stream_plan has the rule).  Here
+//
+// * a workgroup (8 wavefronts, one per CU) takes a contiguous share of all (block, 128 output columns) units, block
+//   by block (stream_plan);
 // * a block's C (up to 64 rows x as much of K as fits 128 KB: all of it up to 32 rows, f16 hi term, both terms
 //   if a row needs them) is copied to LDS once for all of the workgroup's units of the block;
 // * each wavefront then streams its own 16 W2 rows of every unit through a register ring, whole 128-byte
@@ -24,6 +24,7 @@
 // Two terms of C (see moefp8_device.h): a block takes both where a row took exact GEMM1 products or has a
 // measured bound that asks for both (with by_estimate also where the row is of magnitude class 1, the rule of
 // the grouped kernels): at least every row that the 128-row path gives both.
+#pragma once
 #include "moefp8_device.h"
 #include "moefp8_launch.h"
 
@@ -51,6 +52,10 @@ struct StreamLds {
   uint8_t c[kStCBytes + 2 * kStRows * kStPad];
   uint8_t wtr[kStWaves][16 * kBlock];             // transpose buffers
   float sa[32 * 16];                              // row scales of C, [K-block of the pass][16 nt rows]
+  int off[kEGlobal + 1];                          // rows before each expert
+  int first[kEGlobal + 1];                        // cost per column, or chunks, before each expert
+  int budget;                                     // of a chunk (0: shares by cost)
+  int staged;                                     // the LDS-staged units do better
 };
 
 // One pass (K-blocks [kb0, kb0 + n)) over the units [u0, u1) of one block: rows row0 .. row0 + rows - 1 in NT
@@ -226,10 +231,11 @@ __device__ __forceinline__ void stream_pass(const Problem& pb, const Plan& pl, c
 // Blocks of an expert's n rows: the fewest of at most kStRows rows, of about equal height (steps of 16).
 struct StreamBlocks {
   int n, q, r;
+  StreamBlocks() = default;
   __device__ __forceinline__ explicit StreamBlocks(int rows) {
     const int tiles = (rows + 15) / 16;
     n = (tiles + kStRows / 16 - 1) / (kStRows / 16);
-    q = n > 0 ? tiles / n : 0;
+    q = n > 0 ? (int)((float)tiles * __builtin_amdgcn_rcpf((float)n) + 0.001f) : 0;   // (tiles <= 256, n <= 64)
     r = tiles - n * q;
   }
   __device__ __forceinline__ int first(int j) const { return 16 * (j * q + min(j, r)); }
@@ -246,51 +252,151 @@ struct StreamBlocks {
   }
 };
 
-__global__ __launch_bounds__(kStThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm2_stream_kernel(
-    Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int by_estimate) {
-  __shared__ __attribute__((aligned(16))) StreamLds sh;
-  __shared__ int off_s[kEGlobal + 1], first_s[kEGlobal + 1];   // rows, and cost per column, before each expert
-  const int I = pb.I, KB = I / kBlock, NC = pb.H / kStCols, E = pb.E_local;
-  for (int i = threadIdx.x; i <= E; i += kStThreads) off_s[i] = pl.expert_offsets[i];
+// How the workgroups share the units (block, 128 columns).
+//
+// By cost (budget 0): each takes the units that start in its equal part of the cost line, columns innermost, so that
+// it meets one or two blocks and every CU the same work to within one unit.
+//
+// By chunks (budget > 0): each takes one run of units of one block, of at most `budget` cost.  A second block costs a
+// workgroup another start (the decision on C's terms, C's copy to LDS, the first W2 lines: ~4 us, about
+// kStartCost / KB of the cost scale), which a call of a few units per workgroup does not earn back: chosen where the
+// smallest budget whose chunks the grid holds is within one start of the equal part.  Calls by cost alone and so, 32
+// experts, H = 2048, I = 768: T = 65 / 80 / 127 with 8 / 4 / 4 local pairs per token 66.4 -> 61.9, 64.2 -> 58.7, 65.3
+// -> 60.3 us; H = 7168, I = 2048: T = 333 with 1 pair 258.4 -> 257.6.
+constexpr int kStartCost = 13;
+struct StreamChunks {
+  int tall, low;              // units per chunk of the expert's blocks of q + 1 and of q m-tiles
+  int per_tall, per_low, n;   // chunks per block of each height, and of the expert
+  __device__ __forceinline__ StreamChunks(const StreamBlocks& sb, int budget, int NC) {
+    // (quotients of integers below 2^12 in fp32, the offset above the rounding and below the least remainder)
+    auto units = [&](int nt) {
+      return max(1, min(NC, (int)((float)budget * __builtin_amdgcn_rcpf((float)StreamBlocks::cost(nt)) + 0.01f)));
+    };
+    auto chunks = [&](int len) { return (int)((float)(NC + len - 1) * __builtin_amdgcn_rcpf((float)len) + 0.001f); };
+    tall = units(sb.q + 1);
+    low = units(sb.q);
+    per_tall = chunks(tall);
+    per_low = chunks(low);
+    n = sb.r * per_tall + (sb.n - sb.r) * per_low;
+  }
+};
+
+// Fills sh.off and, from the experts' row counts, sh.staged (with staged_ok) and for the stream sh.first and sh.budget
+// (all threads; ends with a barrier).
+//
+// The staged units are taken where their rounds over the grid, (5 KB + 20) of 128-K steps each (KB K-blocks and what a
+// unit costs besides), are no more than the stream's largest share of cost in its padded K-blocks and 40 for its
+// start: a fit to both kernels' times over 202 calls (1 to 256 local experts, H 512 to 8192, I 256 to 4096, T = 128 to
+// 512, 1 to 8 local pairs per token, zipf and all tokens on the same 8 experts), on average 0.5% above the better of
+// the two.  H = 7168, I = 2048, 32 experts, calls by the stream and by the staged units: T = 128, 1 pair 245 and 275 us;
+// 256, 3 pairs 284 and 298; 333, 2 pairs 283 and 295; 333, 4 pairs 325 and 317; 512, 4 pairs 400 and 347; 512, 8
+// pairs 546 and 436; zipf T = 512, 1501 pairs 288 and 243; 2 local experts of H = 4096, I = 1024 74 and 79.
+__device__ __forceinline__ void stream_plan(const Problem& pb, const Plan& pl, StreamLds& sh, bool staged_ok) {
+  const int KB = pb.I / kBlock, NC = pb.H / kStCols, E = pb.E_local, G = (int)gridDim.x;
+  for (int i = threadIdx.x; i <= E; i += kStThreads) sh.off[i] = pl.expert_offsets[i];
   __syncthreads();
   if (threadIdx.x < kWave) {
-    int carry = 0;
-    for (int e0 = 0; e0 < E; e0 += kWave) {
-      const int e = e0 + (int)threadIdx.x;
-      const int c = e < E ? StreamBlocks(off_s[e + 1] - off_s[e]).total() : 0;
-      const int f = carry + wave_exclusive_sum(c);
-      if (e < E) first_s[e] = f;
-      carry = __builtin_amdgcn_readlane(f + c, kWave - 1);
+    constexpr int kPer = kEGlobal / kWave;   // experts per lane
+    const int lane = (int)threadIdx.x;
+    StreamBlocks sb[kPer];
+    int tallest = 0;   // cost of the tallest block
+#pragma unroll
+    for (int i = 0; i < kPer; i++) {
+      if (i * kWave >= E) continue;
+      const int e = min(i * kWave + lane, E - 1);
+      sb[i] = StreamBlocks(i * kWave + lane < E ? sh.off[e + 1] - sh.off[e] : 0);
+      if (sb[i].n > 0) tallest = max(tallest, StreamBlocks::cost(sb[i].r > 0 ? sb[i].q + 1 : sb[i].q));
     }
-    if (threadIdx.x == 0) first_s[E] = carry;
+    // sum over the experts of a whole number below 2^24 in all
+    auto sum = [&](auto&& value) {
+      int v = 0;
+#pragma unroll
+      for (int i = 0; i < kPer; i++)
+        if (i * kWave < E) v += value(sb[i]);
+      return (int)wave_sum_f32((float)v);
+    };
+    const int cost = sum([](const StreamBlocks& b) { return b.total(); });
+    int staged = 0;
+    if (staged_ok && cost > 0) {
+      const int blocks = sum([](const StreamBlocks& b) { return (b.n * b.q + b.r + kGemm2Rows / 16 - 1) / (kGemm2Rows / 16); });
+      const int rounds = (int)((uint32_t)(blocks * (pb.H / 256) + G - 1) / (uint32_t)G);   // of the staged kernel's units over the grid
+      const int padded = (KB + kStDepth - 1) / kStDepth * kStDepth;
+      tallest = (int)wave_max_u32((uint32_t)tallest);
+      staged = max(cost * NC, tallest * G) * padded + 40 * G >= rounds * (5 * KB + 20) * G ? 1 : 0;
+    }
+    int budget = 0;
+    if (!staged) {
+      const int most = (int)((uint32_t)(cost * NC * KB + kStartCost * G) / (uint32_t)(G * KB));
+      for (int b = max(1, (int)((uint32_t)(cost * NC + G - 1) / (uint32_t)G)); b <= most; b++) {
+        if (sum([&](const StreamBlocks& x) { return StreamChunks(x, b, NC).n; }) <= G) {
+          budget = b;
+          break;
+        }
+      }
+      int carry = 0;
+#pragma unroll
+      for (int i = 0; i < kPer; i++) {
+        if (i * kWave >= E) continue;
+        const int c = budget > 0 ? StreamChunks(sb[i], budget, NC).n : sb[i].total();
+        const int f = carry + wave_exclusive_sum(c);
+        if (i * kWave + lane < E) sh.first[i * kWave + lane] = f;
+        carry = __builtin_amdgcn_readlane(f + c, kWave - 1);
+      }
+      if (lane == 0) sh.first[E] = carry;
+    }
+    if (lane == 0) {
+      sh.budget = budget;
+      sh.staged = staged;
+    }
   }
   __syncthreads();
-  // this workgroup's share of the units (block, 128 columns), columns innermost, by cost: the units that
-  // start in [v, v1) of the cost line.  Consecutive shares run on one XCD, so that the blocks of an expert share
-  // its W2 through that XCD's L2.
+}
+
+// This workgroup's units (all threads).
+__device__ __forceinline__ void gemm2_stream_units(const Problem& pb, const Plan& pl, const CHalf8& ch, StreamLds& sh,
+                                                   float* __restrict__ obuf, int by_estimate) {
+  const int I = pb.I, KB = I / kBlock, NC = pb.H / kStCols, E = pb.E_local;
+  // Consecutive shares run on one XCD, so that the blocks of an expert share its W2 through that XCD's L2.
   const int G = (int)gridDim.x, nx = G % 8 == 0 ? 8 : 1;
   const int share = ((int)blockIdx.x % nx) * (G / nx) + (int)blockIdx.x / nx;
-  const int64_t total = (int64_t)first_s[E] * NC;
-  const int v1 = (int)(total * (share + 1) / G);
-  int v = (int)(total * share / G);
+  // by cost, the units that start in [v, v1) of the cost line; by chunks, the chunk in [v, v1) if any (no more than
+  // workgroups, spread over all XCDs)
+  const int budget = uniform(sh.budget), width = budget > 0 ? 1 : NC;
+  // (cost below 2 per row and expert at most 2^11, times 64 columns and 2^9 workgroups)
+  const uint32_t total = (uint32_t)sh.first[E] * width;
+  const int v1 = (int)(total * (share + 1) / (uint32_t)G);
+  int v = (int)(total * share / (uint32_t)G);
   while (v < v1) {
-    // the expert of cost v (the last that starts at or before it; empty ones share their successor's start),
-    // its block there and the block's units in the share
+    // the expert of v (the last that starts at or before it; empty ones share their successor's start), its
+    // block there and the block's units in the share
     int lo = 0, hi = E;
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
-      if (first_s[mid] * NC <= v) lo = mid;
+      if (sh.first[mid] * width <= v) lo = mid;
       else hi = mid;
     }
-    const int e = uniform(lo), n_rows = off_s[e + 1] - off_s[e];
+    const int e = uniform(lo), n_rows = sh.off[e + 1] - sh.off[e];
     const StreamBlocks sb(n_rows);
-    int before;
-    const int j = sb.block_at((v - first_s[e] * NC) / NC, &before);
+    int j, u0, u1;
+    if (budget > 0) {
+      const StreamChunks sc(sb, budget, NC);
+      const int at = v - sh.first[e], tall = sb.r * sc.per_tall;
+      const int per = at < tall ? sc.per_tall : sc.per_low, len = at < tall ? sc.tall : sc.low;
+      const int jj = (at < tall ? at : at - tall) / per, piece = (at < tall ? at : at - tall) - jj * per;
+      j = at < tall ? jj : sb.r + jj;
+      u0 = uniform(piece * len);
+      u1 = uniform(min(NC, piece * len + len));
+      v = v1;
+    } else {
+      int before;
+      j = sb.block_at((v - sh.first[e] * NC) / NC, &before);
+      const int cost = StreamBlocks::cost(j < sb.r ? sb.q + 1 : sb.q), start = (sh.first[e] + before) * NC;
+      u0 = uniform((v - start + cost - 1) / cost);
+      u1 = uniform(min(NC, (v1 - start + cost - 1) / cost));
+      v = start + cost * NC;
+    }
     const int r0 = sb.first(j);
-    const int row0 = uniform(off_s[e] + r0), rows = uniform(min(sb.first(j + 1), n_rows) - r0);
-    const int cost = StreamBlocks::cost(j < sb.r ? sb.q + 1 : sb.q), start = (first_s[e] + before) * NC;
-    const int u0 = uniform((v - start + cost - 1) / cost), u1 = uniform(min(NC, (v1 - start + cost - 1) / cost));
-    v = start + cost * NC;
+    const int row0 = uniform(sh.off[e] + r0), rows = uniform(min(sb.first(j + 1), n_rows) - r0);
     if (u0 >= u1) continue;
     // both terms of C where a row of the block needs them
     bool need = row0 + rows > pl.xrow[e];
@@ -325,12 +431,6 @@ __global__ __launch_bounds__(kStThreads, 1) __attribute__((amdgpu_waves_per_eu(2
 #undef MOEFP8_STREAM
     }
   }
-}
-
-void launch_gemm2_stream(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, bool by_estimate,
-                         hipStream_t stream) {
-  hipLaunchKernelGGL(gemm2_stream_kernel, dim3(num_compute_units()), dim3(kStThreads), 0, stream, pb, pl, ch, obuf,
-                     by_estimate ? 1 : 0);
 }
 
 }  // namespace moefp8

@@ -1,6 +1,6 @@
 // Grouped expert GEMMs for T > 64 (prefill).  Three families: the LDS-staged ones with both operands in LDS
-// (GEMM1 of every call in their range, GEMM2 past kStreamT tokens; their own headers below), gemm2_stream.hip for
-// GEMM2 up to there, and for the shapes outside that range (large_big) the 4-wave ones described here:
+// (GEMM1 of every call in their range, GEMM2 past kStreamT tokens or with many rows per expert; their own headers
+// below), gemm2_stream.h for GEMM2 of a few rows per expert, and for the shapes outside that range (large_big) the 4-wave ones described here:
 // LDS-staged activations, per-wavefront weight streams.
 //
 // A workgroup of 4 wavefronts owns one unit = (m-block of BM = 16*MT rows of one expert,
@@ -29,6 +29,7 @@
 //        and summed per token by the combine kernel.
 #include <type_traits>
 
+#include "gemm2_stream.h"
 #include "moefp8_device.h"
 #include "moefp8_launch.h"
 
@@ -1106,8 +1107,9 @@ struct G2Rows {
 };
 
 // One unit.  Wavefront (wm, wn) computes m-tiles NT wm .. NT wm + NT - 1 (NT = 4, 2 or 1 for
-// blocks whose rows reach past LDS row 64, 32, or not).  kTwo: C's lo term too.
-template <bool kTwo, int NT>
+// blocks whose rows reach past LDS row 64, 32, or not).  kTwo: C's lo term too.  kShort: the kernel's, so that each of
+// the two has instances of its own (shared ones the compiler schedules otherwise: calls of T = 8192 and 14107 +0.4%).
+template <bool kTwo, int NT, bool kShort>
 __device__ __forceinline__ void gemm2_big_unit(const Problem& pb, const Plan& pl, const CHalf8& ch, uint8_t* ring,
                                                uint32_t ring_lds, const float* sw2_s, const float* pw_s, int e,
                                                const G2Rows& rm, int hc, float* __restrict__ obuf, int ocol0,
@@ -1258,9 +1260,15 @@ __device__ __forceinline__ void gemm2_big_unit(const Problem& pb, const Plan& pl
 // Units (m-block, 256 output columns) over GEMM2's own row table (Plan::g2_*): an expert's
 // one-term blocks, then its two-term blocks; the column blocks of output pass `pass` (out_pass),
 // written to O rows of the pass's length from column 0; `pass` also picks the pass's unit queues.
+//
+// kShort (T <= kStreamT, one pass): the stream (gemm2_stream.h) or, with `arg` (the row table is built), these units,
+// whichever the pairs' distribution over the experts asks for (stream_plan).  One kernel for both: a launch that only
+// finds that the other one is wanted costs 3 us of a 250 us call.  Otherwise `arg` is the output pass.
+template <bool kShort>
 __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm2_big_kernel(
-    Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int pass) {
-  __shared__ __attribute__((aligned(16))) uint8_t ring[kB2Stages * kB2Stage];
+    Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int arg) {
+  constexpr int kRing = kB2Stages * kB2Stage, kStream = (int)sizeof(StreamLds);
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kShort && kStream > kRing ? kStream : kRing];
   __shared__ float sw2_s[2 * kBigMaxKB];
   __shared__ float pw_s[kGemm2Rows];
   __shared__ int rowp_s[kGemm2Rows];
@@ -1268,6 +1276,16 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
   __shared__ int g_off[kEGlobal + 1], g_c1[kEGlobal], g_c2[kEGlobal], g_first[kEGlobal + 1];
   const int H = pb.H, I = pb.I, KB = I / kBlock, HB = H / kBlock, E = pb.E_local;
   __shared__ int next_s;
+  const int pass = kShort ? 0 : arg;
+  if constexpr (kShort) {
+    StreamLds& st = *reinterpret_cast<StreamLds*>(ring);
+    stream_plan(pb, pl, st, arg != 0);
+    if (!uniform(st.staged)) {
+      gemm2_stream_units(pb, pl, ch, st, obuf, arg == 0);
+      return;
+    }
+    __syncthreads();   // (`ring` is the staged units' from here)
+  }
   const uint32_t ring_lds = uniform((int)lds_addr(ring));
   const OutPass op = out_pass(pl.info[0], H, o_rows, pass, pl.pair_rows);
   const int hc0 = op.c0 / kB2Cols, hcn = (op.c1 - op.c0) / kB2Cols, ocols = op.ocols;
@@ -1332,7 +1350,7 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     __syncthreads();
     const G2Rows rm{rowp_s, rows};
 #define MOEFP8_G2_UNIT(TWO, NT)                                                                               \
-  gemm2_big_unit<TWO, NT>(pb, pl, ch, ring, ring_lds, sw2_s, pw_s, e, rm, hc, obuf, hcl * kB2Cols, ocols,          \
+  gemm2_big_unit<TWO, NT, kShort>(pb, pl, ch, ring, ring_lds, sw2_s, pw_s, e, rm, hc, obuf, hcl * kB2Cols, ocols,          \
                           op.rows_cap, queues, &next_s, n_units)
     if (two) {
       if (rows <= 32) MOEFP8_G2_UNIT(true, 1);
@@ -1505,7 +1523,13 @@ void launch_gemm2_big(const Problem& pb, const Plan& pl, const CHalf8& ch, float
   const int cus = num_compute_units();
   const int grid = max_units < cus ? max_units : cus;
   if (grid <= 0) return;
-  hipLaunchKernelGGL(gemm2_big_kernel, dim3(grid), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows, pass);
+  hipLaunchKernelGGL(gemm2_big_kernel<false>, dim3(grid), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows, pass);
+}
+
+void launch_gemm2_short(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, int o_rows, bool staged_ok,
+                        hipStream_t stream) {
+  hipLaunchKernelGGL(gemm2_big_kernel<true>, dim3(num_compute_units()), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows,
+                     staged_ok ? 1 : 0);
 }
 
 }  // namespace moefp8

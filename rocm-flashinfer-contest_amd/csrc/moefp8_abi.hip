@@ -498,10 +498,12 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
   }
   mark(3);
   // GEMM2's precision from the C that GEMM1 wrote (the activation stage): per pair, with GEMM2's own row
-  // table, for the LDS-staged kernel; by the stream kernel itself; per m-block for the 4-wave ones
+  // table, for the LDS-staged units; by the stream itself; per m-block for the 4-wave kernels.  Up to kStreamT
+  // tokens GEMM2 chooses between the first two on the device, below kBigT (before which the 4-wave kernels are
+  // the ones to beat: T = 127, 8 local pairs per token 397 us, the stream 295) it always streams.
   const bool stream2 = big && T <= kStreamT && L.o_rows >= L.pmax;
-  if (stream2) {
-    // (the stream kernel decides per block, from the scales of the block that it reads)
+  if (stream2 && T < kBigT) {
+    // (the stream decides per block, from the scales of the block that it reads)
   } else if (big) {
     launch_g2_plan(pb, pl, ch, (int)L.pmax, s);
   } else {
@@ -515,7 +517,7 @@ static int run_impl(const moefp8_args* a, void* workspace, size_t workspace_byte
     // (its two empty launches cost ~7 us per call, measured)
     const int passes = L.o_rows >= L.pmax ? 1 : 2;
     for (int pass = 0; pass < 2; pass++) {
-      if (stream2 && pass == 0) launch_gemm2_stream(pb, pl, ch, obuf, T < kBigT, s);
+      if (stream2 && pass == 0) launch_gemm2_short(pb, pl, ch, obuf, (int)L.o_rows, T >= kBigT, s);
       else if (pass < passes) launch_gemm2_big(pb, pl, ch, obuf, (int)(L.max_blocks2 * (H / 256)), (int)L.o_rows, pass, s);
       mark(5 + 2 * pass);
       if (pass < passes) launch_combine_pass(pl, obuf, a->output, (int)T, H, (int)L.o_rows, pass, s);

@@ -73,7 +73,7 @@ __device__ __forceinline__ void split_f16(float x, float inv, _Float16& hi, _Flo
 // sum |a w|, which this estimate tracks), and pairs above kOneTermRms are grouped together inside
 // their expert and take two terms of C in GEMM2 (kFlagTwoTermC) below 128 tokens and on the
 // 4-wave kernels (from 128 tokens the LDS-staged path decides from the measured C alone: per row in
-// g2_plan_kernel, per block in gemm2_stream_kernel).
+// g2_plan_kernel, per block in gemm2_stream_units).
 constexpr float kPreciseRms = 96.0f;
 constexpr float kOneTermRms = 8.0f;
 constexpr uint8_t kFlagExactProducts = 1;

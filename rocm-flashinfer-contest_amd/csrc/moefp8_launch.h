@@ -198,11 +198,12 @@ __device__ __forceinline__ OutPass out_pass(int P, int H, int o_rows, int pass, 
 void launch_gemm2_big(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, int max_units, int o_rows,
                       int pass, hipStream_t stream);
 
-// GEMM2 for T <= kStreamT on the same C and O (one pass over the columns): C resident in LDS, W2 streamed.
-// With `by_estimate` a block also takes both terms of C for a row of magnitude class 1.
+// GEMM2 for T <= kStreamT on the same C and O (one pass over the columns): C resident in LDS and W2 streamed, or,
+// with `staged_ok` (g2_plan has run), the LDS-staged units, chosen on the device by the experts' pair counts.
+// Without it a block also takes both terms of C for a row of magnitude class 1.
 constexpr int kStreamT = 512;
-void launch_gemm2_stream(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, bool by_estimate,
-                         hipStream_t stream);
+void launch_gemm2_short(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, int o_rows, bool staged_ok,
+                        hipStream_t stream);
 
 void launch_combine(const Plan& pl, const float* obuf, void* out, int T, int H, hipStream_t stream);
 // The combine of output pass `pass` (out_pass).
