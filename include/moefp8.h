@@ -132,10 +132,10 @@ int moefp8_workspace_size(int64_t num_tokens, int32_t num_local_experts, int32_t
 
 /* Kernel family moefp8_run uses for these sizes (host only, no device needed; no counterpart in
  * the reference, whose run() always loops over experts in Python, main.py:218-241):
- * MOEFP8_PATH_SMALL_T (T <= 64: weight-streaming GEMMs), MOEFP8_PATH_GROUPED (64 < T < 128, where
- * the precision of C follows the magnitude estimate too, and shapes outside the LDS-staged GEMMs' range) or
- * MOEFP8_PATH_ROWS128 (the LDS-staged GEMMs, precision of C from C itself, from T = 128), or a negative
- * status. */
+ * MOEFP8_PATH_SMALL_T (T <= 64: weight-streaming GEMMs), MOEFP8_PATH_ROWS128 (T > 64: GEMM1 staged in
+ * LDS; GEMM2 streamed up to T = 127, streamed or LDS-staged by the experts' rows up to T = 512, LDS-staged
+ * past it) or MOEFP8_PATH_GROUPED (T > 64, shapes that the LDS-staged kernels do not take: 4-wave grouped
+ * GEMMs), or a negative status. */
 #define MOEFP8_PATH_SMALL_T 0
 #define MOEFP8_PATH_GROUPED 1
 #define MOEFP8_PATH_ROWS128 2
@@ -163,7 +163,7 @@ int moefp8_run(const moefp8_args* args, void* workspace, size_t workspace_bytes,
  * static device array of MOEFP8_NOALLOC_SCRATCH_BYTES (64 MiB) per device that loads the library,
  * held until the process ends; sizes whose moefp8_workspace_size() exceeds it return
  * MOEFP8_ERR_SCRATCH_LIMIT before any launch (at H = 7168, I = 2048 it covers every T <= 226 for
- * E_local 8, 32 or 256: the small-T and grouped paths and the 128-row path up to T = 226).  The
+ * E_local 8, 32 or 256: the small-T path, and the large-T ones up to T = 226).  The
  * call itself allocates nothing.  Every call on a device shares that device's array: calls that overlap on
  * one device (different streams, or other host threads) race and must be serialised by the
  * caller; calls on one stream are ordered by it.  Each call initialises what it reads. */

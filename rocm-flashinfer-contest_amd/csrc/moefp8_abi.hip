@@ -24,7 +24,7 @@ constexpr int64_t kDecodeMaxT = 64;
 // even with a few rows per expert this streams each weight slice once per block, with GEMM2's streaming kernel
 // 207 / 218 / 241 / 240 us at T = 65 / 80 / 100 / 127 against 246 / 258 / 278 / 276 us for the 4-wave
 // kernels below.  Those (blocks of 16 * large_mt(T) rows) remain for shapes the staged kernels do not take.
-// kBigT is where moefp8_path's MOEFP8_PATH_ROWS128 begins (per-pair precision of C in GEMM2).
+// From kBigT on GEMM2's precision follows the measured C alone, and up to kStreamT it may take the staged units.
 constexpr int64_t kBigT = 128;
 // The staged kernels address their DMA sources with 32-bit per-lane byte offsets from a
 // wave-uniform base: hidden rows (token x H, GEMM1) and C rows (pair x 2I, GEMM2).  Shapes whose
@@ -259,9 +259,8 @@ int moefp8_path(int64_t num_tokens, int32_t num_local_experts, int32_t hidden_si
   const int rc = check_sizes(num_tokens, num_local_experts, hidden_size, intermediate_size);
   if (rc) return rc;
   if (num_tokens <= kDecodeMaxT) return MOEFP8_PATH_SMALL_T;
-  return num_tokens >= kBigT && large_big(num_tokens, num_local_experts, hidden_size, intermediate_size)
-             ? MOEFP8_PATH_ROWS128
-             : MOEFP8_PATH_GROUPED;
+  return large_big(num_tokens, num_local_experts, hidden_size, intermediate_size) ? MOEFP8_PATH_ROWS128
+                                                                                    : MOEFP8_PATH_GROUPED;
 }
 
 int moefp8_output_passes(int64_t num_tokens, int32_t num_local_experts, int32_t hidden_size,

@@ -74,7 +74,7 @@ def test_workspace_size(lib):
     assert passes(8192, 32, 7168, 2048, pmax) == 2
     assert passes(4681, 32, 7168, 2048, 8 * 4681) == 1          # 4681 * 8 * 7168 * 4 B < 1 GiB: all rows
     assert passes(4682, 32, 7168, 2048, 8 * 4682) == 2
-    assert passes(4682, 32, 384, 2048, 8 * 4682) == 1           # not the 128-row path (H % 256)
+    assert passes(4682, 32, 384, 2048, 8 * 4682) == 1           # not the LDS-staged path (H % 256)
     assert passes(64, 32, 7168, 2048, 512) == 1
     assert passes(-1, 32, 7168, 2048, 0) == -2
     assert passes(16, 32, 7168, 2048, -1) == -2
@@ -165,7 +165,7 @@ def test_missing_library_raises(tmp_path):
 
 
 def test_path_dispatch_bounds(lib):
-    """moefp8_path: T <= 64 streams weights; from T = 128 the 128-row kernels run unless their
+    """moefp8_path: T <= 64 streams weights; past it the LDS-staged kernels run unless their
     32-bit DMA offsets could wrap (T x H >= 2^31, or Pmax x 2I >= 2^32 with Pmax = T x min(8,
     E_local)), or H is not a multiple of 256, or a K range exceeds 64 blocks; those shapes take
     the 4-wave grouped kernels (64-bit addresses)."""
@@ -173,8 +173,9 @@ def test_path_dispatch_bounds(lib):
     H, I = 7168, 2048
     assert p(1, 32, H, I) == _abi.PATH_SMALL_T
     assert p(64, 32, H, I) == _abi.PATH_SMALL_T
-    assert p(65, 32, H, I) == _abi.PATH_GROUPED
-    assert p(127, 32, H, I) == _abi.PATH_GROUPED
+    assert p(65, 32, H, I) == _abi.PATH_ROWS128
+    assert p(127, 32, H, I) == _abi.PATH_ROWS128
+    assert p(65, 32, 384, I) == _abi.PATH_GROUPED
     assert p(128, 32, H, I) == _abi.PATH_ROWS128
     assert p(8192, 32, H, I) == _abi.PATH_ROWS128
     # Pmax x 2I at the 2^32 edge (E_local >= 8: Pmax = 8T)
@@ -186,7 +187,7 @@ def test_path_dispatch_bounds(lib):
     t = (1 << 31) // H
     assert p(t, 1, H, 128) == _abi.PATH_ROWS128
     assert p(t + 1, 1, H, 128) == _abi.PATH_GROUPED
-    # shapes the 128-row kernels do not take
+    # shapes the LDS-staged kernels do not take
     assert p(4096, 32, 384, I) == _abi.PATH_GROUPED         # H % 256 != 0
     assert p(4096, 32, 128 * 65 * 2, I) == _abi.PATH_GROUPED  # H / 128 > 64
     assert p(4096, 32, H, 128 * 65) == _abi.PATH_GROUPED    # I / 128 > 64

@@ -152,15 +152,17 @@ REDUCED = [
     (2500, 32, 256, 128, 0),
     (2048, 32, 256, 128, 0),        # one-workgroup permutation, two rounds of 4 token blocks
     (1100, 32, 256, 128, 0),        # ... and a second round with one block
-    (2100, 16, 512, 256, 0),        # 128-row blocks with 4 K-blocks
+    (2100, 16, 512, 256, 0),        # LDS-staged GEMMs with 4 and 2 K-blocks
     (16, 32, 512, 256, 32),         # expert-parallel rank 1 (one routing group)
     (40, 32, 256, 128, 240),        # rank owning experts 240..271: half past the last expert
     (500, 32, 256, 128, 32),
     (300, 32, 512, 256, 240),
-    (127, 16, 512, 256, 0),         # last T of the 4-wave grouped GEMMs
-    (128, 16, 512, 256, 0),         # first T of the 128-row GEMMs
-    (129, 64, 256, 128, 192),       # 128-row GEMMs, 64 local experts, two routing groups
-    (600, 8, 768, 384, 0),          # 128-row GEMMs with 6 and 3 K-blocks
+    (127, 16, 512, 256, 0),         # last T at which GEMM2 always streams
+    (128, 16, 512, 256, 0),         # first T at which it may take the LDS-staged units
+    (129, 64, 256, 128, 192),       # 64 local experts, two routing groups
+    (600, 8, 768, 384, 0),          # LDS-staged GEMMs with 6 and 3 K-blocks
+    (127, 16, 640, 256, 0),         # 4-wave grouped GEMMs, 32-row blocks
+    (1600, 16, 640, 1152, 0),       # the same, 64-row blocks, 9 K-blocks in GEMM2
 ]
 
 
@@ -330,8 +332,9 @@ def test_golden_fixtures_full_path():
 
 @pytest.mark.parametrize("T,E_local,H,I,shared,path", [(300, 16, 512, 256, False, 2), (1100, 32, 256, 128, False, 2),
                                                          (300, 16, 512, 256, True, 2), (16, 32, 512, 256, False, 0),
-                                                         (40, 16, 256, 128, True, 0), (100, 32, 512, 256, False, 1),
-                                                         (100, 32, 512, 256, True, 1)])
+                                                         (40, 16, 256, 128, True, 0), (100, 32, 512, 256, False, 2),
+                                                         (100, 32, 512, 256, True, 2), (100, 32, 640, 256, False, 1),
+                                                         (100, 32, 640, 256, True, 1)])
 def test_rows_without_local_pair_overwrite_stale_output(T, E_local, H, I, shared, path):
     """Rows of tokens without a local pair: exact zeros (or bf16 of the shared row), written by the
     small-T GEMM2's epilogue (path 0) or by the combine (paths 1 and 2).  The output buffer is
@@ -502,16 +505,24 @@ def test_full_path_workloads(name, full_weights):
         assert int(counts.sum()) >= 1 and float(ref32.abs().max()) > 0.0
 
 
-def test_full_path_grouped_kernels_at_full_size(full_weights):
-    """T = 96 at H = 7168, I = 2048 takes the grouped 16*MT-row kernels (64 < T < 128), whose
-    two-term GEMM2 mode the flags launch drives: routing, permutation and output against the
-    oracle."""
+def columns(weights, H):
+    """The weights of the same experts on their first H hidden columns (a multiple of 128)."""
+    w13, s13, w2, s2 = weights
+    return (w13[:, :, :H].contiguous(), s13[:, :, :H // 128].contiguous(), w2[:, :H].contiguous(),
+            s2[:, :H // 128].contiguous())
+
+
+@pytest.mark.parametrize("T,H,path", [(96, 7168, 2), (96, 7040, 1), (1600, 7040, 1)])
+def test_full_path_between_decode_and_prefill_at_full_size(full_weights, T, H, path):
+    """T = 96 at H = 7168, I = 2048 takes the LDS-staged GEMM1 and GEMM2's stream; at H = 7040, which is no multiple of
+    256, the grouped 16*MT-row kernels (MT = 2, from T = 1536 on 4), whose two-term GEMM2 mode the flags launch drives:
+    routing, permutation and output against the oracle."""
     from moe_fp8 import _abi
     lib = _abi.load()
-    assert lib.moefp8_path(96, 32, 7168, 2048) == _abi.PATH_GROUPED
-    wl = W.Workload("grouped_t96", 96, 196)
-    w_dev, w_cpu = full_weights
-    act = W.make_activations(wl, device=DEV)
+    assert lib.moefp8_path(T, 32, H, 2048) == path
+    wl = W.Workload(f"t{T}_h{H}", T, 100 + T)
+    w_dev, w_cpu = (w if H == 7168 else columns(w, H) for w in full_weights)
+    act = W.make_activations(wl, device=DEV, H=H)
     act_cpu = to_cpu(act)
     dbg = {}
     out = moe_fp8.run(*act, *w_dev, 0, W.RSF, debug=dbg)
@@ -522,8 +533,8 @@ def test_full_path_grouped_kernels_at_full_size(full_weights):
     assert np.array_equal(dbg["expert_offsets"].cpu().numpy(), offsets)
     assert np.array_equal(dbg["permuted_tokens"].cpu().numpy()[: offsets[-1]], ptok)
     ref32, _ = O.moe_forward(*act_cpu, *w_cpu, 0, W.RSF)
-    err = assert_close(out, ref32, "grouped_t96")
-    print(f"[full] grouped_t96 P={int(counts.sum())} max_abs_err={err:.3e}", flush=True)
+    err = assert_close(out, ref32, wl.name)
+    print(f"[full] {wl.name} P={int(counts.sum())} max_abs_err={err:.3e}", flush=True)
 
 
 def test_full_path_four_row_tile_on_two_way_split(full_weights):

@@ -25,6 +25,7 @@ import torch
 
 import moe_oracle as O
 import moe_fp8
+from moe_fp8 import _abi
 from moe_fp8 import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -47,19 +48,19 @@ def dequant_row(w13c, s13, e, r):
     return torch.from_numpy(q * np.repeat(s13[e, r // 128].numpy(), 128))
 
 
-def build(kind, T, seed, w_cpu):
+def build(kind, T, seed, w_cpu, h=H):
     g = torch.Generator().manual_seed(seed)
     logits = torch.randn(T, 256, generator=g)
     bias = (torch.randn(256, generator=g) * 0.1).to(torch.bfloat16)
     chosen = torch.stack([torch.randperm(E, generator=g)[:8] for _ in range(T)])   # 8 local experts per token
     logits.scatter_add_(1, chosen, torch.full((T, 8), 6.0))
-    x = torch.randn(T, H, generator=g)
+    x = torch.randn(T, h, generator=g)
     w13c, s13 = w_cpu[0], w_cpu[1]
     if kind in ("aligned", "both", "aligned_block"):
         rows = 4 if kind == "aligned_block" else 1
         for t in range(T):
             n = 2 + t % 2
-            a = torch.zeros(H)
+            a = torch.zeros(h)
             for e in chosen[t, :n].tolist():
                 # `rows` consecutive C columns j.. inside one 128-column block: only the block's
                 # largest element lands exactly on the split's 448, the others round in f16
@@ -72,7 +73,7 @@ def build(kind, T, seed, w_cpu):
         x *= torch.exp(torch.randn(T, 1, generator=g) * 1.5)         # log-normal row amplitudes
     if kind in ("outliers", "both"):
         for t in range(T):
-            ch = torch.randperm(H, generator=g)[: 2 + t % 7]
+            ch = torch.randperm(h, generator=g)[: 2 + t % 7]
             x[t, ch] *= 100.0
     hs, hss = W.quantize_rows_1x128(x)
     return logits, bias, hs, hss
@@ -117,7 +118,7 @@ def check(w_dev, w_cpu, act):
     assert not bad
 
 
-@pytest.mark.parametrize("T", [48, 100, 400])   # the small-T, grouped 16*MT-row and 128-row paths
+@pytest.mark.parametrize("T", [48, 100, 400])   # the small-T path, GEMM2 streamed, and streamed or LDS-staged
 def test_structured_weights_flat_w2(flat_w2_weights, T):
     print(f"[structured] flat_w2 T={T}", flush=True)
     w_dev, w_cpu = flat_w2_weights
@@ -125,7 +126,7 @@ def test_structured_weights_flat_w2(flat_w2_weights, T):
 
 
 @pytest.mark.parametrize("kind", ["aligned", "aligned_block", "outliers", "both", "amplified"])
-@pytest.mark.parametrize("T", [48, 100, 400])   # the small-T, grouped 16*MT-row and 128-row paths
+@pytest.mark.parametrize("T", [48, 100, 400])   # the small-T path, GEMM2 streamed, and streamed or LDS-staged
 def test_structured_activations(weights, kind, T):
     print(f"[structured] {kind} T={T}", flush=True)
     w_dev, w_cpu = weights
@@ -149,3 +150,16 @@ def test_structured_activations(weights, kind, T):
     for b in bad[:10]:
         print("   t=%d h=%d fp32 %.5f fp64 %.5f HIP %.5f" % b, flush=True)
     assert not bad
+
+
+@pytest.mark.parametrize("kind,T", [("aligned", 100), ("aligned_block", 100), ("both", 100), ("amplified", 100),
+                                    ("flat_w2", 100), ("aligned", 1600), ("flat_w2", 1600)])
+def test_structured_four_wave_kernels(weights, flat_w2_weights, kind, T):
+    """The same on H = 7040, no multiple of 256: the grouped 16*MT-row kernels (MT = 2; from T = 1536 on 4), whose
+    blocks take two terms of C by the flags launch's measured rule."""
+    print(f"[structured] four-wave {kind} T={T}", flush=True)
+    h = 7040
+    assert _abi.load().moefp8_path(T, E, h, I) == _abi.PATH_GROUPED
+    w_dev, w_cpu = (tuple(x.contiguous() for x in (w13[:, :, :h], s13[:, :, :h // 128], w2[:, :h], s2[:, :h // 128]))
+                    for w13, s13, w2, s2 in (flat_w2_weights if kind == "flat_w2" else weights))
+    check(w_dev, w_cpu, build("amplified" if kind == "flat_w2" else kind, T, 7200 + T + len(kind), w_cpu, h))

@@ -24,10 +24,12 @@ def inputs(T, E_local, H, I, seed):
     return [logits.to(DEV), bias.to(DEV), hs.to(DEV), hss.to(DEV)]
 
 
-# (T, E_local, H, I, path): the decode, grouped 16*MT-row and 128-row paths, and the headline
-# decode size at full width
-CASES = [(48, 16, 512, 256, _abi.PATH_SMALL_T), (100, 16, 512, 256, _abi.PATH_GROUPED),
-         (400, 16, 512, 256, _abi.PATH_ROWS128), (16, 32, 7168, 2048, _abi.PATH_SMALL_T)]
+# (T, E_local, H, I, path): the decode path, the LDS-staged one (GEMM2 streamed, either way, staged), the 4-wave
+# kernels (32- and 64-row blocks), and the headline decode size at full width
+CASES = [(48, 16, 512, 256, _abi.PATH_SMALL_T), (100, 16, 512, 256, _abi.PATH_ROWS128),
+         (400, 16, 512, 256, _abi.PATH_ROWS128), (1600, 16, 512, 256, _abi.PATH_ROWS128),
+         (100, 16, 640, 256, _abi.PATH_GROUPED), (1600, 16, 640, 256, _abi.PATH_GROUPED),
+         (16, 32, 7168, 2048, _abi.PATH_SMALL_T)]
 
 
 @pytest.mark.parametrize("T,E_local,H,I,path", CASES)
