@@ -1265,8 +1265,7 @@ __device__ __forceinline__ void gemm2_big_unit(const Problem& pb, const Plan& pl
 // whichever the pairs' distribution over the experts asks for (stream_plan).  One kernel for both: a launch that only
 // finds that the other one is wanted costs 3 us of a 250 us call.  Otherwise `arg` is the output pass.
 template <bool kShort>
-__global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm2_big_kernel(
-    Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int arg) {
+__device__ __forceinline__ void gemm2_big(Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int arg) {
   constexpr int kRing = kB2Stages * kB2Stage, kStream = (int)sizeof(StreamLds);
   __shared__ __attribute__((aligned(16))) uint8_t ring[kShort && kStream > kRing ? kStream : kRing];
   __shared__ float sw2_s[2 * kBigMaxKB];
@@ -1365,6 +1364,15 @@ __global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2
     // next_s is written
     __syncthreads();
   }
+}
+
+__global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm2_big_kernel(
+    Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int pass) {
+  gemm2_big<false>(pb, pl, ch, obuf, o_rows, pass);
+}
+__global__ __launch_bounds__(kBgThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm2_short_kernel(
+    Problem pb, Plan pl, CHalf8 ch, float* __restrict__ obuf, int o_rows, int staged_ok) {
+  gemm2_big<true>(pb, pl, ch, obuf, o_rows, staged_ok);
 }
 
 // ------------------------------------------------------------------------------------------ flags
@@ -1523,12 +1531,12 @@ void launch_gemm2_big(const Problem& pb, const Plan& pl, const CHalf8& ch, float
   const int cus = num_compute_units();
   const int grid = max_units < cus ? max_units : cus;
   if (grid <= 0) return;
-  hipLaunchKernelGGL(gemm2_big_kernel<false>, dim3(grid), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows, pass);
+  hipLaunchKernelGGL(gemm2_big_kernel, dim3(grid), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows, pass);
 }
 
 void launch_gemm2_short(const Problem& pb, const Plan& pl, const CHalf8& ch, float* obuf, int o_rows, bool staged_ok,
                         hipStream_t stream) {
-  hipLaunchKernelGGL(gemm2_big_kernel<true>, dim3(num_compute_units()), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows,
+  hipLaunchKernelGGL(gemm2_short_kernel, dim3(num_compute_units()), dim3(kBgThreads), 0, stream, pb, pl, ch, obuf, o_rows,
                      staged_ok ? 1 : 0);
 }
 
