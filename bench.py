@@ -217,7 +217,7 @@ def measure(wl, weights, steps, warmup, flush):
     else:
         ach = k_flops / (k_us * 1e-6) / 1e12
         roof = dict(bound="mfma", achieved=ach, peak=FP8_PEAK / 1e12, unit="TFLOP/s", frac=ach / (FP8_PEAK / 1e12))
-    kernel = STAGE_KERNELS[(dom, "decode" if T <= 64 else "large")]
+    kernel = STAGE_KERNELS[(dom, "decode" if T <= 64 else "chunk" if T <= 512 else "large")]
     tr = traced_us(kernel, wl.name)
     roof.update(kernel=kernel, kernel_us=k_us, algorithmic_bytes=k_bytes, algorithmic_flops=k_flops,
                 traffic=measured_traffic(kernel, wl.name), trace_us=tr,
@@ -231,9 +231,10 @@ def measure(wl, weights, steps, warmup, flush):
     return res
 
 
-# The library's kernel names per bench stage ("gemm1" / "gemm2"), by path: decode (T <= 64), and
-# the 128-row grouped GEMMs of the large path.
+# The library's kernel names per bench stage ("gemm1" / "gemm2"): decode (T <= 64), chunks (up to T = 512, whose
+# GEMM2 streams or takes the LDS-staged units) and the LDS-staged grouped GEMMs past them.
 STAGE_KERNELS = {("gemm1", "decode"): "gemm1_decode_kernel", ("gemm2", "decode"): "gemm2_decode_kernel",
+                 ("gemm1", "chunk"): "gemm1_big_kernel", ("gemm2", "chunk"): "gemm2_short_kernel",
                  ("gemm1", "large"): "gemm1_big_kernel", ("gemm2", "large"): "gemm2_big_kernel"}
 PROFILES = ROOT / "profiles"
 

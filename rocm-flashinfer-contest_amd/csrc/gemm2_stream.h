@@ -318,8 +318,10 @@ __device__ __forceinline__ void stream_plan(const Problem& pb, const Plan& pl, S
     const int cost = sum([](const StreamBlocks& b) { return b.total(); });
     int staged = 0;
     if (staged_ok && cost > 0) {
-      const int blocks = sum([](const StreamBlocks& b) { return (b.n * b.q + b.r + kGemm2Rows / 16 - 1) / (kGemm2Rows / 16); });
-      const int rounds = (int)((uint32_t)(blocks * (pb.H / 256) + G - 1) / (uint32_t)G);   // of the staged kernel's units over the grid
+      // rounds of the staged units over the grid
+      constexpr int kTiles = kGemm2Rows / 16;
+      const int blocks = sum([](const StreamBlocks& b) { return (b.n * b.q + b.r + kTiles - 1) / kTiles; });
+      const int rounds = (int)((uint32_t)(blocks * (pb.H / 256) + G - 1) / (uint32_t)G);
       const int padded = (KB + kStDepth - 1) / kStDepth * kStDepth;
       tallest = (int)wave_max_u32((uint32_t)tallest);
       staged = max(cost * NC, tallest * G) * padded + 40 * G >= rounds * (5 * KB + 20) * G ? 1 : 0;
@@ -362,7 +364,7 @@ __device__ __forceinline__ void gemm2_stream_units(const Problem& pb, const Plan
   // by cost, the units that start in [v, v1) of the cost line; by chunks, the chunk in [v, v1) if any (no more than
   // workgroups, spread over all XCDs)
   const int budget = uniform(sh.budget), width = budget > 0 ? 1 : NC;
-  // (cost below 2 per row and expert at most 2^11, times 64 columns and 2^9 workgroups)
+  // (at most 512 m-tiles of cost 2 in 64 columns: 32 bits hold the products)
   const uint32_t total = (uint32_t)sh.first[E] * width;
   const int v1 = (int)(total * (share + 1) / (uint32_t)G);
   int v = (int)(total * share / (uint32_t)G);

@@ -1,7 +1,7 @@
 // Grouped expert GEMMs for T > 64 (prefill).  Three families: the LDS-staged ones with both operands in LDS
 // (GEMM1 of every call in their range, GEMM2 past kStreamT tokens or with many rows per expert; their own headers
-// below), gemm2_stream.h for GEMM2 of a few rows per expert, and for the shapes outside that range (large_big) the 4-wave ones described here:
-// LDS-staged activations, per-wavefront weight streams.
+// below), gemm2_stream.h for GEMM2 of a few rows per expert, and for the shapes outside that range (large_big) the
+// 4-wave ones described here: LDS-staged activations, per-wavefront weight streams.
 //
 // A workgroup of 4 wavefronts owns one unit = (m-block of BM = 16*MT rows of one expert,
 // block of 128 output columns).  Each wavefront streams its own 32 or 64 weight rows

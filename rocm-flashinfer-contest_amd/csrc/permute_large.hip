@@ -5,8 +5,8 @@
 //   place  per block, from all blocks' counts (staged in LDS; up to kSelfBlocks blocks count for
 //          themselves): every bucket's total and this block's prefix of it, hence the bucket and
 //          expert offsets; each pair's rank inside its bucket in token order then gives its row,
-//          the rank inside its expert alone its canonical row.  Block 0 also writes the offsets and the m-block table of the grouped
-//          GEMMs.  (A one-workgroup scan launch between the two took 5-7 us plus a launch
+//          the rank inside its expert alone its canonical row.  Block 0 also writes the offsets and the m-block
+//          table of the grouped GEMMs.  (A one-workgroup scan launch between the two took 5-7 us plus a launch
 //          boundary at T = 1024-8192; every block redoing the sums it needs costs it one round of
 //          loads.)
 //

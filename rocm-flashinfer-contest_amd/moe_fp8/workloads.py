@@ -16,6 +16,7 @@ routed scaling 2.5):
   local experts 0-31 (routing plus the zero output only), so
 * ``decode_t1_local`` / ``decode_t4_local`` take the first seed 100+T+k (k >= 1) whose routing
   gives local work: seed 102 (1 pair, 1 active expert) and seed 105 (2 pairs, 2 experts).
+* ``chunk``     T=333, seed 333 (a chunked-prefill step: GEMM2 streams).
 * ``prefill``   T=1024, seed 1024.
 * ``large``     T=8192, seed 8192; per-token hidden amplitude exp(z), z~N(0,1).
 * ``skewed``    T=5000, seed 5000; Zipf(s=1.2) expert popularity over a seeded
@@ -58,6 +59,7 @@ def workloads():
         w[f"decode_t{T}"] = Workload(f"decode_t{T}", T, 100 + T)
     w["decode_t1_local"] = Workload("decode_t1_local", 1, 102)
     w["decode_t4_local"] = Workload("decode_t4_local", 4, 105)
+    w["chunk_t333"] = Workload("chunk_t333", 333, 333)
     w["prefill_t1024"] = Workload("prefill_t1024", 1024, 1024)
     w["large_t8192"] = Workload("large_t8192", 8192, 8192, hidden_dist="lognormal")
     w["skewed_t5000"] = Workload("skewed_t5000", 5000, 5000, routing="zipf")
