@@ -284,28 +284,32 @@ struct StreamChunks {
 // Fills sh.off and, from the experts' row counts, sh.staged (with staged_ok) and for the stream sh.first and sh.budget
 // (all threads; ends with a barrier).
 //
-// The staged units are taken where their rounds over the grid, (5 KB + 20) of 128-K steps each (KB K-blocks and what a
-// unit costs besides), are no more than the stream's largest share of cost in its padded K-blocks and 40 for its
-// start: a fit to both kernels' times over 202 calls (1 to 256 local experts, H 512 to 8192, I 256 to 4096, T = 128 to
-// 512, 1 to 8 local pairs per token, zipf and all tokens on the same 8 experts), on average 0.5% above the better of
-// the two.  H = 7168, I = 2048, 32 experts, calls by the stream and by the staged units: T = 128, 1 pair 245 and 275 us;
-// 256, 3 pairs 284 and 298; 333, 2 pairs 283 and 295; 333, 4 pairs 325 and 317; 512, 4 pairs 400 and 347; 512, 8
-// pairs 546 and 436; zipf T = 512, 1501 pairs 288 and 243; 2 local experts of H = 4096, I = 1024 74 and 79.
+// The staged units are taken where their rounds over the grid, (5 KB + 24) of 128-K steps each (KB K-blocks and what a
+// unit costs besides), are no more than the stream's largest share of cost in its padded K-blocks and 48 for its
+// start, an expert with rows of two-term C costing half more: a fit to both kernels' times over 262 calls (8 to 256 local
+// experts, H 512 to 8192, I 256 to 4096, T = 128 to 512, 1 to 8 local pairs per token, normal and log-normal
+// tokens, zipf and all tokens on the same 8 experts), on average 0.3% above the better of the two.  H = 7168, I = 2048,
+// 32 experts, calls by the stream and by the staged units: T = 128, 1 pair 245 and 275 us; 256, 3 pairs 284 and 298;
+// 333, 2 pairs 283 and 295; 333, 4 pairs 325 and 317; 512, 4 pairs 400 and 347; 512, 8 pairs 546 and 436; zipf T = 512,
+// 1501 pairs 288 and 243.  256 experts, I = 256, log-normal, T = 256 391 and 488 (each expert has blocks of both kinds);
+// 16 experts of H = 8192, I = 4096, log-normal, T = 128, 4 pairs 463 and 405.
 __device__ __forceinline__ void stream_plan(const Problem& pb, const Plan& pl, StreamLds& sh, bool staged_ok) {
   const int KB = pb.I / kBlock, NC = pb.H / kStCols, E = pb.E_local, G = (int)gridDim.x;
+  constexpr int kPer = kEGlobal / kWave;   // experts per lane
+  int2 ctl[kPer];                          // one- and two-term rows of each
+  if (staged_ok) {
+#pragma unroll
+    for (int i = 0; i < kPer; i++) ctl[i] = reinterpret_cast<const int2*>(pl.g2_ctl)[min(i * kWave + lane_id(), E - 1)];
+  }
   for (int i = threadIdx.x; i <= E; i += kStThreads) sh.off[i] = pl.expert_offsets[i];
   __syncthreads();
   if (threadIdx.x < kWave) {
-    constexpr int kPer = kEGlobal / kWave;   // experts per lane
     const int lane = (int)threadIdx.x;
     StreamBlocks sb[kPer];
-    int tallest = 0;   // cost of the tallest block
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      if (i * kWave >= E) continue;
       const int e = min(i * kWave + lane, E - 1);
-      sb[i] = StreamBlocks(i * kWave + lane < E ? sh.off[e + 1] - sh.off[e] : 0);
-      if (sb[i].n > 0) tallest = max(tallest, StreamBlocks::cost(sb[i].r > 0 ? sb[i].q + 1 : sb[i].q));
+      if (i * kWave < E) sb[i] = StreamBlocks(i * kWave + lane < E ? sh.off[e + 1] - sh.off[e] : 0);
     }
     // sum over the experts of a whole number below 2^24 in all
     auto sum = [&](auto&& value) {
@@ -318,13 +322,22 @@ __device__ __forceinline__ void stream_plan(const Problem& pb, const Plan& pl, S
     const int cost = sum([](const StreamBlocks& b) { return b.total(); });
     int staged = 0;
     if (staged_ok && cost > 0) {
-      // rounds of the staged units over the grid
-      constexpr int kTiles = kGemm2Rows / 16;
-      const int blocks = sum([](const StreamBlocks& b) { return (b.n * b.q + b.r + kTiles - 1) / kTiles; });
-      const int rounds = (int)((uint32_t)(blocks * (pb.H / 256) + G - 1) / (uint32_t)G);
+      // of this lane's experts: the staged units' blocks; twice the cost, three times with two-term rows, and the tallest
+      // block's
+      int blocks = 0, weighted = 0, tallest = 0;
+#pragma unroll
+      for (int i = 0; i < kPer; i++) {
+        if (i * kWave >= E || sb[i].n == 0) continue;
+        const int w = ctl[i].y > 0 ? 3 : 2;
+        blocks += (ctl[i].x + kGemm2Rows - 1) / kGemm2Rows + (ctl[i].y + kGemm2Rows - 1) / kGemm2Rows;
+        weighted += w * sb[i].total();
+        tallest = max(tallest, w * StreamBlocks::cost(sb[i].r > 0 ? sb[i].q + 1 : sb[i].q));
+      }
+      const int units = (int)wave_sum_f32((float)blocks) * (pb.H / 256);
+      const int rounds = (int)((uint32_t)(units + G - 1) / (uint32_t)G);   // of the staged units over the grid
       const int padded = (KB + kStDepth - 1) / kStDepth * kStDepth;
-      tallest = (int)wave_max_u32((uint32_t)tallest);
-      staged = max(cost * NC, tallest * G) * padded + 40 * G >= rounds * (5 * KB + 20) * G ? 1 : 0;
+      const int share = max((int)wave_sum_f32((float)weighted) * NC, (int)wave_max_u32((uint32_t)tallest) * G);
+      staged = share * padded + 96 * G >= 2 * rounds * (5 * KB + 24) * G ? 1 : 0;
     }
     int budget = 0;
     if (!staged) {

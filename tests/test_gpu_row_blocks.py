@@ -38,22 +38,25 @@ def gemm1_height(counts, exact, I, slots):
     return 128 if rounds[128] <= rounds[160] else 160
 
 
-def gemm2_kind(counts, H, I, T, slots):
-    """How GEMM2 takes a call of 64 < T <= 512: LDS-staged units, or the stream by chunks or by cost."""
+def gemm2_kind(counts, exact, H, I, T, slots):
+    """How GEMM2 takes a call of 64 < T <= 512: LDS-staged units, or the stream by chunks or by cost (rows take two
+    terms of C where their products are exact)."""
     KB, NC = I // 128, H // 128
     unit_cost = lambda nt: 2 if nt <= 1 else 2 * nt - 1
-    blocks = []                                  # (m-tiles, blocks) of the stream
-    for n in counts:
+    blocks, staged, weighted, tallest = [], 0, 0, 0      # blocks: (m-tiles, number) of the stream's
+    for n, n2 in zip(counts, exact):
         tiles = cdiv(n, 16)
         k = cdiv(tiles, 4)
-        if k:
-            blocks += [(tiles // k + 1, tiles % k), (tiles // k, k - tiles % k)]
-    blocks = [b for b in blocks if b[1]]
+        mine = [b for b in ((tiles // k + 1, tiles % k), (tiles // k, k - tiles % k)) if b[1]] if k else []
+        w = 3 if n2 else 2
+        blocks += mine
+        staged += cdiv(n - n2, 128) + cdiv(n2, 128)
+        weighted += w * sum(unit_cost(nt) * c for nt, c in mine)
+        tallest = max([tallest] + [w * unit_cost(nt) for nt, _ in mine])
     cost = sum(unit_cost(nt) * k for nt, k in blocks)
     if T >= 128 and cost:
-        rounds = cdiv(sum(cdiv(n, 128) for n in counts) * (H // 256), slots)
-        tallest = max(unit_cost(nt) for nt, _ in blocks)
-        if max(cost * NC, tallest * slots) * cdiv(KB, 8) * 8 + 40 * slots >= rounds * (5 * KB + 20) * slots:
+        rounds = cdiv(staged * (H // 256), slots)
+        if max(weighted * NC, tallest * slots) * cdiv(KB, 8) * 8 + 96 * slots >= 2 * rounds * (5 * KB + 24) * slots:
             return "staged"
     most = (cost * NC * KB + 13 * slots) // (slots * KB)
     for b in range(max(1, cdiv(cost * NC, slots)), most + 1):
@@ -160,15 +163,16 @@ def test_blocks_of_160_rows(counts, exact):
     (127, 512, 2176, (33, 49, 17, 28), (0, 49, 0, 1), "chunks"),
     (127, 256, 2048, (127,), (40,), "cost"),
     (127, 2048, 384, (17, 16, 1) * 3, (0, 16, 1) * 3, "chunks"),
-    (200, 2048, 1024, (2, 2), (0, 2), "chunks"),
     (200, 2048, 2048, (16,) * 8, (0, 1) * 4, "chunks"),
-    (500, 512, 2048, (15, 16, 17) * 10, (0, 16, 1) * 10, "cost"),
+    (200, 2048, 2048, (5,) * 20, (0, 2) * 10, "cost"),
+    (500, 512, 2048, (15, 16, 17) * 10, (0,) * 30, "cost"),
+    (500, 512, 2048, (15, 16, 17) * 10, (0, 16, 1) * 10, "staged"),   # two blocks per expert, but two terms in the stream
     (512, 2048, 2048, (128, 127, 129, 128), (0, 127, 1, 33), "staged"),
     (512, 512, 256, (159, 160, 161, 5), (0, 0, 33, 5), "staged")])
 def test_gemm2_kinds(T, H, I, counts, exact, kind):
     """Each way that GEMM2 takes a call of up to 512 tokens, as its rule on the experts' rows chooses."""
     print(f"[gemm2] T={T} H={H} I={I} {counts[:4]} exact {exact[:4]} {kind}", flush=True)
-    assert gemm2_kind(counts, H, I, T, compute_units()) == kind
+    assert gemm2_kind(counts, exact, H, I, T, compute_units()) == kind
     check(counts, exact, T, H, I, seed=T + H + I)
 
 
