@@ -49,19 +49,28 @@ __device__ __forceinline__ int exact_blocks(const LargePermArgs& a, int n2) {
 // The blocks over an expert's class 0/1 rows, in steps of 32 rows: n of them, the first r of q + 1 steps and
 // the others of q (the last ends with the rows).  Without `mixed`, blocks of rows_a rows.  With it the fewest
 // blocks of at most rows_a rows, of about equal height: 260 rows as 160 + 100 and not 160 + 96 + 4, since
-// a block streams its expert's whole weight slice however short it is.  Folded exact rows count as one step of
-// the last block, whose height then stays within kMixedRows (q <= 4; q >= 2, so it keeps class 0/1 rows too).
+// a block streams its expert's whole weight slice however short it is.  Folded exact rows belong to the last block.
+// Cut loosely they take a step of their own, and blocks that would be full with it are one more: a shorter last block,
+// as an exact m-tile costs GEMM1 about three others.  Cut tightly, those of one m-tile take the free half of the last
+// step if there is one, and blocks of kBigRowsLow may be full: no more blocks than a cut every 128 rows has.  Either
+// way the last block's height stays within kMixedRows (q <= 4), and it keeps class 0/1 rows too.
 struct RowBlocks {
   int n, q, r;
   __device__ __forceinline__ int first(int j) const { return 32 * (j * q + min(j, r)); }
 };
-__device__ __forceinline__ RowBlocks row_blocks(const LargePermArgs& a, int rows_a, int n01, int n2) {
-  if (!a.mixed) return RowBlocks{(n01 + rows_a - 1) / rows_a, rows_a / 32, 0};
-  const bool fold = folds_exact(a, n01, n2), high = rows_a == kBigRows;
-  const int steps = (n01 + 31) / 32 + (fold ? 1 : 0);
+// A cut: the largest block height, and how folded rows are cut.
+struct RowCut {
+  int rows_a;
+  bool tight;
+};
+__device__ __forceinline__ RowBlocks row_blocks(const LargePermArgs& a, RowCut cut, int n01, int n2) {
+  if (!a.mixed) return RowBlocks{(n01 + cut.rows_a - 1) / cut.rows_a, cut.rows_a / 32, 0};
+  const bool fold = folds_exact(a, n01, n2), high = cut.rows_a == kBigRows;
+  const bool half = cut.tight && n2 <= 16 && ((n01 - 1) & 31) < 16;
+  const int steps = (n01 + 31) / 32 + (fold && !half ? 1 : 0);
   constexpr int kHigh = kBigRows / 32, kLow = kBigRowsLow / 32;   // (divisions by constants)
   int n = high ? (steps + kHigh - 1) / kHigh : (steps + kLow - 1) / kLow;
-  if (fold && steps == n * (high ? kHigh : kLow)) n++;
+  if (fold && (high || !cut.tight) && steps == n * (high ? kHigh : kLow)) n++;
   const int q = n > 0 ? steps / n : 0;
   return RowBlocks{n, q, steps - n * q};
 }
@@ -221,25 +230,36 @@ __device__ __forceinline__ int upper_bound(const int* v, int n, int x) {
 // An expert's blocks are consecutive, so the units that stream its weights run close together in
 // time and share them through L2.  With `write`, also the path's global tables.
 //
-// Returns the largest block height (meaningful with `write` alone: only the tables depend on it).  With `mixed` it
-// is kBigRows, or kBigRowsLow where that takes GEMM1 no more rounds of units over its workgroups: the same number
-// of rounds of shorter units.  GEMM1's calls at zipf routing:
-// T = 1000 234 us at 160, 225 at 128 (as many rounds); T = 1500 256 and 285 us (one round more at 128).
-__device__ int expert_offsets(const LargePermArgs& a, const int* tot, int* eoff, int* emt, int* eb1, bool write) {
+// Returns the cut (meaningful with `write` alone: only the tables depend on it).  With `mixed` it is, of the two heights
+// cut tightly and loosely, the one that takes GEMM1 the fewest rounds of units over its workgroups, and of those
+// the one of most blocks: the same number of rounds of shorter units.  GEMM1's calls at zipf routing:
+// T = 1000 234 us at 160, 225 at 128 (as many rounds); T = 1500 256 and 285 us (one round more at 128).  GEMM1 with
+// log-normal tokens, tight and loose, us: T = 700, 4 local pairs 196 and 237 (a round more); 400, 8 pairs 197 and 233;
+// 3000, 1 pair 253 and 240 (as many rounds); 1024, 4 pairs 268 and 253; cut every 128 rows 207, 211, 278 and 296.
+__device__ RowCut expert_offsets(const LargePermArgs& a, const int* tot, int* eoff, int* emt, int* eb1, bool write) {
   const int E = a.E_local, lane = lane_id();
-  int rows_a = a.rows_a;
+  RowCut cut = {a.rows_a, false};
   if (a.mixed && write) {
-    int high = 0, low = 0, rest = 0;
+    constexpr int kCuts = 4;
+    const RowCut cuts[kCuts] = {{kBigRowsLow, false}, {kBigRowsLow, true}, {kBigRows, false}, {kBigRows, true}};
+    int blocks[kCuts] = {};
     for (int e = lane; e < E; e += kWave) {
       const int n01 = tot[kClasses * e] + tot[kClasses * e + 1], n2 = tot[kClasses * e + 2];
-      high += row_blocks(a, kBigRows, n01, n2).n;
-      low += row_blocks(a, kBigRowsLow, n01, n2).n;
-      rest += folds_exact(a, n01, n2) ? 0 : exact_blocks(a, n2);
+      const int rest = folds_exact(a, n01, n2) ? 0 : exact_blocks(a, n2);
+#pragma unroll
+      for (int c = 0; c < kCuts; c++) blocks[c] += row_blocks(a, cuts[c], n01, n2).n + rest;
     }
-    // (counts below 2^24: exact in fp32)
-    const int uh = (int)wave_sum_f32((float)(high + rest)) * a.units;
-    const int ul = (int)wave_sum_f32((float)(low + rest)) * a.units;
-    if ((ul + a.slots - 1) / a.slots <= (uh + a.slots - 1) / a.slots) rows_a = kBigRowsLow;
+    int best = 0, most = 0;
+#pragma unroll
+    for (int c = 0; c < kCuts; c++) {
+      // (counts below 2^24: exact in fp32)
+      const int n = (int)wave_sum_f32((float)blocks[c]), rounds = (n * a.units + a.slots - 1) / a.slots;
+      if (c == 0 || rounds < best || (rounds == best && n > most)) {
+        best = rounds;
+        most = n;
+        cut = cuts[c];
+      }
+    }
   }
   int carry = 0, carry_mt = 0, carry_1 = 0, carry_act = 0;
   for (int e0 = 0; e0 < E; e0 += kWave) {
@@ -247,7 +267,7 @@ __device__ int expert_offsets(const LargePermArgs& a, const int* tot, int* eoff,
     const int n0 = e < E ? tot[kClasses * e] : 0, n1 = e < E ? tot[kClasses * e + 1] : 0;
     const int n2 = e < E ? tot[kClasses * e + 2] : 0, n = n0 + n1 + n2;
     const int mt = (n + 15) / 16;
-    const int ba = row_blocks(a, rows_a, n0 + n1, n2).n;
+    const int ba = row_blocks(a, cut, n0 + n1, n2).n;
     const int bx = folds_exact(a, n0 + n1, n2) ? 0 : exact_blocks(a, n2);
     const int b1 = ba + bx;
     const int pn = wave_exclusive_sum(n), pmt = wave_exclusive_sum(mt);
@@ -285,16 +305,16 @@ __device__ int expert_offsets(const LargePermArgs& a, const int* tot, int* eoff,
       a.info[6] = carry_mt;             // 16-row m-tiles
     }
   }
-  return rows_a;
+  return cut;
 }
 
 // The m-block table {expert, first row, rows, flags} and each block's expert group (all threads).
-__device__ void write_mblocks(const LargePermArgs& a, int rows_a, const int* tot, const int* eoff, const int* eb1) {
+__device__ void write_mblocks(const LargePermArgs& a, RowCut cut, const int* tot, const int* eoff, const int* eb1) {
   const int E = a.E_local;
   for (int g = threadIdx.x; g < eb1[E]; g += blockDim.x) {
     const int e = upper_bound(eb1, E + 1, g) - 1, j = g - eb1[e];
     const int c0 = tot[kClasses * e], c01 = c0 + tot[kClasses * e + 1], n = eoff[e + 1] - eoff[e];
-    const RowBlocks rb = row_blocks(a, rows_a, c01, n - c01);
+    const RowBlocks rb = row_blocks(a, cut, c01, n - c01);
     const int ba = rb.n;
     if (j < ba) {
       const int r0 = rb.first(j), rows = min(rb.first(j + 1), c01) - r0;
@@ -336,7 +356,7 @@ __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a)
   __shared__ int tot[kEGlobal * kClasses], pre[kEGlobal * kClasses];
   __shared__ int eoff[kEGlobal + 1], emt[kEGlobal + 1], eb1[kEGlobal + 1];
   __shared__ int stage[kSelf ? 1 : kPlaceLdsInts];
-  __shared__ int rows_a;   // largest block height
+  __shared__ RowCut cut;
   const int E = a.E_local, E3 = E * kClasses, tid = threadIdx.x, wave = tid >> 6;
   const int t = blockIdx.x * kBlkTokens + tid;
   const bool in = t < a.T;
@@ -349,8 +369,8 @@ __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a)
   else bucket_sums(a, blockIdx.x, tot, pre, stage);
   const bool first = blockIdx.x == 0;
   if (wave == 0) {
-    const int r = expert_offsets(a, tot, eoff, emt, eb1, first);
-    if (tid == 0) rows_a = r;
+    const RowCut r = expert_offsets(a, tot, eoff, emt, eb1, first);
+    if (tid == 0) cut = r;
   }
   if (first) {
     // the grouped GEMMs' unit queues and the 128-row GEMM2's row-table counters start at zero
@@ -358,7 +378,7 @@ __global__ __launch_bounds__(kBlkTokens) void perm_place_kernel(LargePermArgs a)
     for (int i = tid; a.g2_ctl && i < 2 * E; i += kBlkTokens) a.g2_ctl[i] = 0;
   }
   __syncthreads();
-  if (first) write_mblocks(a, rows_a, tot, eoff, eb1);
+  if (first) write_mblocks(a, cut, tot, eoff, eb1);
   int bk[kTopK], ek[kTopK], rb[kTopK], re[kTopK];
 #pragma unroll
   for (int k = 0; k < kTopK; k++) {

@@ -24,18 +24,22 @@ def compute_units():
     return torch.cuda.get_device_properties(0).multi_processor_count
 
 
-def gemm1_height(counts, exact, I, slots):
-    """The largest block height of the staged GEMM1: 160 rows where that saves a round of units, else 128."""
-    rounds = {}
-    for height in (160, 128):
+def gemm1_cut(counts, exact, I, slots):
+    """The staged GEMM1's largest block height, and whether an expert's folded exact rows are cut tightly: of the four the
+    one of fewest rounds of units, and of those the one of most blocks."""
+    best = None
+    for height, tight in ((128, False), (128, True), (160, False), (160, True)):
         blocks = 0
         for n, n2 in zip(counts, exact):
             n01, fold = n - n2, 1 <= n2 <= 32 and n > n2
-            steps = cdiv(n01, 32) + fold
+            steps = cdiv(n01, 32) + (fold and not (tight and n2 <= 16 and (n01 - 1) % 32 < 16))
             k = cdiv(steps, height // 32)
-            blocks += k + (fold and steps == k * (height // 32)) + (0 if fold else cdiv(n2, 32))
-        rounds[height] = cdiv(blocks * (I // 128), slots)
-    return 128 if rounds[128] <= rounds[160] else 160
+            blocks += k + (fold and (height == 160 or not tight) and steps == k * (height // 32))
+            blocks += 0 if fold else cdiv(n2, 32)
+        rank = (cdiv(blocks * (I // 128), slots), -blocks)
+        if best is None or rank < best[0]:
+            best = (rank, height, tight)
+    return best[1:]
 
 
 def gemm2_kind(counts, exact, H, I, T, slots):
@@ -118,6 +122,7 @@ def test_rows_per_expert(counts, T):
 @pytest.mark.parametrize("T", [0, 1100])
 @pytest.mark.parametrize("counts,exact", [((1, 2, 16, 17), (1, 1, 16, 16)), ((33, 48, 49, 64), (1, 16, 17, 32)),
                                           ((97, 128, 129, 160), (1, 17, 32, 32)), ((161, 193, 225, 300), (33, 32, 16, 40)),
+                                          ((128, 129, 113, 98), (16, 16, 17, 1)), ((96, 104, 256, 273), (1, 8, 16, 17)),
                                           ((290, 320, 40, 35), (1, 32, 40, 3))])
 def test_exact_rows_per_expert(counts, exact, T):
     """1 to 32 exact rows fold into an expert's last block, more get blocks of their own."""
@@ -143,16 +148,22 @@ def test_token_block_edges(T):
     check(counts, (T // 9, 0, 1, 3), T, 512, 256, seed=T)
 
 
-@pytest.mark.parametrize("counts,exact", [((129, 144, 145, 159, 160), (0,) * 5), ((128, 131, 133, 160, 190), (33, 40, 33, 64, 33)),
-                                          ((112, 113, 129, 129, 160), (16, 17, 1, 32, 40)),
-                                          ((33, 97, 160, 270, 320), (1, 32, 0, 17, 0))])
-def test_blocks_of_160_rows(counts, exact):
-    """32 experts of eight GEMM1 units per block: a second round of units if any expert took two blocks.  Class 0/1
-    rows up to 160 in one block, beside exact-product blocks (more than 32 exact rows) and mixed ones (their step of
-    32 rows makes the fifth of an expert's steps a second block)."""
-    counts, exact = (counts * 7)[:32], (exact * 7)[:32]
-    print(f"[160 rows] {counts[:5]} exact {exact[:5]}", flush=True)
-    assert gemm1_height(counts, exact, 1024, compute_units()) == 160
+@pytest.mark.parametrize("counts,exact,cut", [
+    ((129, 144, 145, 159, 160), (0,) * 5, (160, False)),
+    ((128, 131, 133, 160, 190), (33, 40, 33, 64, 33), (160, False)),      # exact-product blocks beside them
+    ((112, 144, 113, 160, 129, 145), (16, 0, 17, 0, 0, 0), (160, False)),
+    ((96, 320, 160, 300), (32, 32, 0, 0), (160, False)),
+    ((98, 160, 112, 150), (1, 0, 15, 0), (160, True)),                    # folded in the free half of a step
+    ((128, 288, 160, 129, 300), (16, 16, 0, 0, 31), (160, True)),
+    ((320, 288, 304, 160), (32, 16, 0, 0), (160, True)),
+    ((108, 100, 128, 112), (8, 10, 16, 1), (128, True)),
+    ((128, 128, 96, 104), (16, 1, 32, 8), (128, False))])
+def test_gemm1_cuts(counts, exact, cut):
+    """32 experts of eight GEMM1 units per block, so that the rounds of units differ between the cuts: blocks of up to 160
+    or 128 class 0/1 rows, folded exact rows tightly or loosely."""
+    counts, exact = (counts * 8)[:32], (exact * 8)[:32]
+    print(f"[cuts] {counts[:6]} exact {exact[:6]} {cut}", flush=True)
+    assert gemm1_cut(counts, exact, 1024, compute_units()) == cut
     check(counts, exact, sum(counts), 256, 1024, seed=sum(counts) + sum(exact))
 
 
