@@ -284,11 +284,13 @@ struct StreamChunks {
 // Fills sh.off and, from the experts' row counts, sh.staged (with staged_ok) and for the stream sh.first and sh.budget
 // (all threads; ends with a barrier).
 //
-// The staged units are taken where their rounds over the grid, (5 KB + 24) of 128-K steps each (KB K-blocks and what a
-// unit costs besides), are no more than the stream's largest share of cost in its padded K-blocks and 48 for its
-// start, an expert with rows of two-term C costing half more: a fit to both kernels' times over 262 calls (8 to 256 local
-// experts, H 512 to 8192, I 256 to 4096, T = 128 to 512, 1 to 8 local pairs per token, normal and log-normal
-// tokens, zipf and all tokens on the same 8 experts), on average 0.3% above the better of the two.  H = 7168, I = 2048,
+// The staged units are taken where their rounds over the grid, (5 KB + 20) of 128-K steps each (KB K-blocks and what a
+// unit costs besides), are no more than the stream's equal share of cost in its padded K-blocks, a quarter more
+// for an expert with rows of two-term C, and 8 for its start and 32 for each further pass over K of its tallest block: a
+// fit to both kernels' times over 418 calls (1 to 256 local experts, H 512 to 8192, I 256 to 4096, T = 128 to 512, 1 to
+// 8 local pairs per token, normal and log-normal tokens, zipf; the weights not in a cache), on average 0.3% above the
+// better of the two.  Calls of one round lean to the stream: 16 experts, H = 2048, I = 1024, T = 512 61 us against 65,
+// zipf T = 256, 6 pairs 48 and 53; 8 experts, H = 2048, I = 2048, T = 512 76 and 82.  H = 7168, I = 2048,
 // 32 experts, calls by the stream and by the staged units: T = 128, 1 pair 245 and 275 us; 256, 3 pairs 284 and 298;
 // 333, 2 pairs 283 and 295; 333, 4 pairs 325 and 317; 512, 4 pairs 400 and 347; 512, 8 pairs 546 and 436; zipf T = 512,
 // 1501 pairs 288 and 243.  256 experts, I = 256, log-normal, T = 256 391 and 488 (each expert has blocks of both kinds);
@@ -322,22 +324,23 @@ __device__ __forceinline__ void stream_plan(const Problem& pb, const Plan& pl, S
     const int cost = sum([](const StreamBlocks& b) { return b.total(); });
     int staged = 0;
     if (staged_ok && cost > 0) {
-      // of this lane's experts: the staged units' blocks; twice the cost, three times with two-term rows, and the tallest
-      // block's
-      int blocks = 0, weighted = 0, tallest = 0;
+      // of this lane's experts: the staged units' blocks; four times the cost, five with two-term rows; and the most
+      // planes of C in a block
+      int blocks = 0, weighted = 0, planes = 0;
 #pragma unroll
       for (int i = 0; i < kPer; i++) {
         if (i * kWave >= E || sb[i].n == 0) continue;
-        const int w = ctl[i].y > 0 ? 3 : 2;
+        const bool two = ctl[i].y > 0;
         blocks += (ctl[i].x + kGemm2Rows - 1) / kGemm2Rows + (ctl[i].y + kGemm2Rows - 1) / kGemm2Rows;
-        weighted += w * sb[i].total();
-        tallest = max(tallest, w * StreamBlocks::cost(sb[i].r > 0 ? sb[i].q + 1 : sb[i].q));
+        weighted += (two ? 5 : 4) * sb[i].total();
+        planes = max(planes, (two ? 2 : 1) * (sb[i].r > 0 ? sb[i].q + 1 : sb[i].q));
       }
       const int units = (int)wave_sum_f32((float)blocks) * (pb.H / 256);
       const int rounds = (int)((uint32_t)(units + G - 1) / (uint32_t)G);   // of the staged units over the grid
-      const int padded = (KB + kStDepth - 1) / kStDepth * kStDepth;
-      const int share = max((int)wave_sum_f32((float)weighted) * NC, (int)wave_max_u32((uint32_t)tallest) * G);
-      staged = share * padded + 96 * G >= 2 * rounds * (5 * KB + 24) * G ? 1 : 0;
+      const int padded = (KB + kStDepth - 1) / kStDepth * kStDepth, share = (int)wave_sum_f32((float)weighted) * NC;
+      const uint32_t kc = (uint32_t)stream_kc((int)wave_max_u32((uint32_t)planes));
+      const int again = (int)(((uint32_t)KB + kc - 1) / kc) - 1;   // passes over K after the first
+      staged = share * padded + 4 * (8 + 32 * again) * G >= 4 * rounds * (5 * KB + 20) * G ? 1 : 0;
     }
     int budget = 0;
     if (!staged) {

@@ -47,20 +47,21 @@ def gemm2_kind(counts, exact, H, I, T, slots):
     terms of C where their products are exact)."""
     KB, NC = I // 128, H // 128
     unit_cost = lambda nt: 2 if nt <= 1 else 2 * nt - 1
-    blocks, staged, weighted, tallest = [], 0, 0, 0      # blocks: (m-tiles, number) of the stream's
+    blocks, staged, weighted, planes = [], 0, 0, 0       # blocks: (m-tiles, number) of the stream's
     for n, n2 in zip(counts, exact):
         tiles = cdiv(n, 16)
         k = cdiv(tiles, 4)
         mine = [b for b in ((tiles // k + 1, tiles % k), (tiles // k, k - tiles % k)) if b[1]] if k else []
-        w = 3 if n2 else 2
         blocks += mine
         staged += cdiv(n - n2, 128) + cdiv(n2, 128)
-        weighted += w * sum(unit_cost(nt) * c for nt, c in mine)
-        tallest = max([tallest] + [w * unit_cost(nt) for nt, _ in mine])
+        weighted += (5 if n2 else 4) * sum(unit_cost(nt) * c for nt, c in mine)
+        planes = max([planes] + [(2 if n2 else 1) * nt for nt, _ in mine])
     cost = sum(unit_cost(nt) * k for nt, k in blocks)
     if T >= 128 and cost:
         rounds = cdiv(staged * (H // 256), slots)
-        if max(weighted * NC, tallest * slots) * cdiv(KB, 8) * 8 + 96 * slots >= 2 * rounds * (5 * KB + 24) * slots:
+        fit, deep = 128 * 1024 // (planes * 16 * 256), 8 if planes <= 4 else 4      # K-blocks of C in LDS, in whole rings
+        again = cdiv(KB, fit - fit % deep) - 1
+        if weighted * NC * cdiv(KB, 8) * 8 + 4 * (8 + 32 * again) * slots >= 4 * rounds * (5 * KB + 20) * slots:
             return "staged"
     most = (cost * NC * KB + 13 * slots) // (slots * KB)
     for b in range(max(1, cdiv(cost * NC, slots)), most + 1):
@@ -177,9 +178,15 @@ def test_gemm1_cuts(counts, exact, cut):
     (200, 2048, 2048, (16,) * 8, (0, 1) * 4, "chunks"),
     (200, 2048, 2048, (5,) * 20, (0, 2) * 10, "cost"),
     (500, 512, 2048, (15, 16, 17) * 10, (0,) * 30, "cost"),
-    (500, 512, 2048, (15, 16, 17) * 10, (0, 16, 1) * 10, "staged"),   # two blocks per expert, but two terms in the stream
-    (512, 2048, 2048, (128, 127, 129, 128), (0, 127, 1, 33), "staged"),
-    (512, 512, 256, (159, 160, 161, 5), (0, 0, 33, 5), "staged")])
+    (500, 512, 2048, (15, 16, 17) * 10, (0, 16, 1) * 10, "cost"),     # (the staged units would be two blocks per expert)
+    (512, 512, 256, (159, 160, 161, 5), (0, 0, 33, 5), "chunks"),     # one round of units
+    (512, 2048, 256, (33, 17, 49) * 5, (0, 5, 49) * 5, "staged"),
+    (512, 4096, 512, (129, 160, 145), (0, 33, 5), "staged"),
+    (500, 2048, 640, (33,) * 15, (0,) * 15, "staged"),
+    (256, 512, 4096, (80, 17, 3, 128), (0, 17, 0, 64), "staged"),     # eight passes over K in the stream
+    (440, 512, 2048, (65, 80) * 3, (0,) * 6, "chunks"),               # two, four with both terms
+    (440, 512, 2048, (65, 80) * 3, (0, 33) * 3, "staged"),
+    (512, 2048, 2048, (128, 127, 129, 128), (0, 127, 1, 33), "staged")])
 def test_gemm2_kinds(T, H, I, counts, exact, kind):
     """Each way that GEMM2 takes a call of up to 512 tokens, as its rule on the experts' rows chooses."""
     print(f"[gemm2] T={T} H={H} I={I} {counts[:4]} exact {exact[:4]} {kind}", flush=True)
